@@ -40,26 +40,9 @@ static_assert(TILE_RING % 2 == 0, "the ring slots and the two LDS buffers advanc
 #define QD_TILE_GROUP_M 8
 #endif
 constexpr int TILE_GROUP_M = QD_TILE_GROUP_M;
-#ifndef QD_BIG_GROUP_M
-#define QD_BIG_GROUP_M 4  // 256 x 256 tiles: 4 M blocks per group (8: 1-4 % slower at 32768 rows)
-#endif
-constexpr int BIG_GROUP_M = QD_BIG_GROUP_M;
-#ifndef QD_TILE8
-#define QD_TILE8 1        // 8-wave 128 x 128 tiles below the 256 x 256 kernel's row count
-#endif
-#ifndef QD_BIG_MIN_M
-#define QD_BIG_MIN_M 1024
-#endif
 #ifndef QD_TILE_ROWS
 #define QD_TILE_ROWS 1     // all-rows kernel at 65..256 rows
 #endif
-#ifndef QD_BIG_ARGMAX_MIN_M
-#define QD_BIG_ARGMAX_MIN_M 129   // LM head rows from which the 256 x 256 argmax tile is used
-#endif
-#ifndef QD_BIG_EPIS
-#define QD_BIG_EPIS 7     // epilogues (bit EPI_NONE, EPI_RES, EPI_SWIGLU) that take the big tile
-#endif
-
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
@@ -313,160 +296,6 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(
   }
 }
 
-// ------------------------------------------------------------------ 128 x 128 tiles, 8 waves
-// The same tile, K stages, LDS layout, remap and split-K as gemm_tile_kernel, with 8 waves per
-// workgroup instead of 4: wave (wm, wn) owns activation rows 64 wm .. x weight rows 32 wn ..
-// (4 x 2 MFMA tiles), so each SIMD holds two waves of one workgroup (four when two workgroups
-// share a CU) to overlap one wave's loads and LDS traffic with another's MFMAs.  SwiGLU: a
-// wave's 32 weight rows are 16 gate rows and the 16 up rows of the same outputs.
-struct Stage8 {
-  uint4 w0, w1, x0, x1;
-};
-
-template <int EPI, bool SPLIT>
-__global__ __launch_bounds__(512, 2) void gemm_tile8_kernel(
-    const bf16_t* __restrict__ X, int64_t x_stride, int M, const bf16_t* __restrict__ W, int N,
-    int K, int mblocks, int nblocks, int ks_per, bf16_t* out, int64_t out_stride, const bf16_t* res,
-    int64_t res_stride, float* part) {
-  static_assert(EPI != EPI_ARGMAX, "the LM head keeps the 4-wave kernel");
-  __shared__ TileLds sm;
-  const int total = gridDim.x, h = blockIdx.x;
-  const int xq = total >> 3, xr = total & 7, xcd = h & 7, slot = h >> 3;
-  const int L = xcd < xr ? xcd * (xq + 1) + slot : xr * (xq + 1) + (xcd - xr) * xq + slot;
-  const int tiles = mblocks * nblocks;
-  const int split = L / tiles;
-  const int Lt = L - split * tiles;
-  const int group = Lt / (TILE_GROUP_M * nblocks);
-  const int first = group * TILE_GROUP_M;
-  const int gm = min(TILE_GROUP_M, mblocks - first);
-  const int rr = Lt - first * nblocks;
-  const int mb = first + rr % gm;
-  const int nb = rr / gm;
-
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int c = lane & 15, q = lane >> 4;
-  const int wn = wave & 3, wm = wave >> 2;
-  const int64_t m0 = (int64_t)mb * TM;
-  const int ksteps = K / TK;
-  const int kbeg = split * ks_per;
-  const int kend = min(ksteps, kbeg + ks_per);
-
-  // staging: thread tid moves unit tid % 8 of LDS rows r0 + 64 i (r0 = tid / 8, i < 2) of both
-  // tiles.  Weight row of LDS row R: nb*128 + R, or for SwiGLU nb*64 + 16 (R / 32) + R % 16,
-  // plus N when (R / 16) is odd (the up rows)
-  const int r0 = tid >> 3, unit0 = tid & 7;
-  const int Nrows = EPI == EPI_SWIGLU ? 2 * N : N;
-  auto wrow_of = [&](int i) -> int64_t {
-    const int R = r0 + 64 * i;
-    const int64_t wr = EPI == EPI_SWIGLU
-                           ? (int64_t)nb * 64 + 16 * (R >> 5) + (R & 15) + (((R >> 4) & 1) ? N : 0)
-                           : (int64_t)nb * TN + R;
-    return (wr < Nrows ? wr : Nrows - 1) * (K / 8) + unit0;          // in uint4 units
-  };
-  auto xrow_of = [&](int i) -> int64_t {
-    const int64_t xm = m0 + r0 + 64 * i;
-    return (xm < M ? xm : M - 1) * (x_stride / 8) + unit0;
-  };
-  const uint4* W4 = reinterpret_cast<const uint4*>(W);
-  const uint4* X4 = reinterpret_cast<const uint4*>(X);
-  const int64_t wo0 = wrow_of(0), wo1 = wrow_of(1), xo0 = xrow_of(0), xo1 = xrow_of(1);
-  uint4* lw0 = &sm.w[0][r0 * 8 + (unit0 ^ (r0 & 7))];              // + 512: rows + 64
-  uint4* lx0 = &sm.x[0][r0 * 8 + (unit0 ^ (r0 & 7))];
-  Stage8 st0, st1;
-  auto load = [&](Stage8& st, int ks) {
-    const int64_t kk = (int64_t)(ks < kend ? ks : kend - 1) * 8;
-    st.w0 = ld_stream(W4 + wo0 + kk);
-    st.w1 = ld_stream(W4 + wo1 + kk);
-    st.x0 = X4[xo0 + kk];
-    st.x1 = X4[xo1 + kk];
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto store = [&](const Stage8& st, int buf) {
-    lw0[buf * (TN * 8)] = st.w0;
-    lw0[buf * (TN * 8) + 512] = st.w1;
-    lx0[buf * (TM * 8)] = st.x0;
-    lx0[buf * (TM * 8) + 512] = st.x1;
-  };
-  f32x4_t acc[2][4];
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int fa = (32 * wn + c) * 8, fb = (64 * wm + c) * 8;           // fragment rows (+ 128 t)
-  auto compute = [&](int buf) {
-#pragma unroll
-    for (int s_ = 0; s_ < 2; ++s_) {
-      const int u_ = (4 * s_ + q) ^ (c & 7);
-      uint4 a_[2], b_[4];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) a_[t] = sm.w[buf][fa + 128 * t + u_];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) b_[t] = sm.x[buf][fb + 128 * t + u_];
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
-          acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(a_[nt]), as_bf8(b_[mt]),
-                                                                acc[nt][mt], 0, 0, 0);
-    }
-  };
-  // as gemm_tile_kernel: stage s in LDS buffer s & 1, loads of stages s + 1, s + 2 in flight
-  load(st0, kbeg);
-  load(st1, kbeg + 1);
-  store(st0, 0);
-  lds_barrier();
-  int ks = kbeg;
-  for (; ks + 1 < kend; ks += 2) {
-    load(st0, ks + 2);
-    compute(0);
-    store(st1, 1);
-    lds_barrier();
-    load(st1, ks + 3);
-    compute(1);
-    store(st0, 0);
-    lds_barrier();
-  }
-  if (ks < kend) compute(0);
-
-  // epilogue: lane (c, q) of acc[nt][mt] holds weight rows 4 q + r of tile nt = output columns
-  // n .. n + 3 of activation row m = m0 + 64 wm + 16 mt + c
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int64_t m = m0 + 64 * wm + 16 * mt + c;
-    if (m >= M) continue;
-    if constexpr (SPLIT) {
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const int64_t n = (int64_t)nb * TN + 32 * wn + 16 * nt + 4 * q;
-        *reinterpret_cast<f32x4_t*>(part + ((int64_t)split * M + m) * N + n) = acc[nt][mt];
-      }
-    } else if constexpr (EPI == EPI_SWIGLU) {
-      const int64_t n = (int64_t)nb * 64 + 16 * wn + 4 * q;
-      float y[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) y[r] = silu_rbf(rbf(acc[0][mt][r])) * rbf(acc[1][mt][r]);
-      *reinterpret_cast<uint2*>(out + m * out_stride + n) = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-    } else {
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const int64_t n = (int64_t)nb * TN + 32 * wn + 16 * nt + 4 * q;
-        float y[4];
-        if constexpr (EPI == EPI_RES) {
-          const uint2 rv = *reinterpret_cast<const uint2*>(res + m * res_stride + n);
-          y[0] = bflo(rv.x) + rbf(acc[nt][mt][0]);
-          y[1] = bfhi(rv.x) + rbf(acc[nt][mt][1]);
-          y[2] = bflo(rv.y) + rbf(acc[nt][mt][2]);
-          y[3] = bfhi(rv.y) + rbf(acc[nt][mt][3]);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) y[r] = acc[nt][mt][r];
-        }
-        *reinterpret_cast<uint2*>(out + m * out_stride + n) = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-      }
-    }
-  }
-}
-
 // Sum of the split partials in split order + epilogue (store / residual); one thread per four
 // consecutive output columns.
 template <int EPI>
@@ -504,258 +333,6 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __r
     for (int r = 0; r < 4; ++r) y[r] = a[r];
   }
   *reinterpret_cast<uint2*>(out + m * out_stride + n) = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-}
-
-// ------------------------------------------------------------------ 256 x 256 tiles (prefill)
-// At prefill row counts (thousands of activation rows) the 128 x 128 tile above moves every
-// weight and activation byte through L1 once per 128 rows of the other operand (6.4 GB of
-// L1->L2 reads per 4096-row gate/up launch, a third of them L2 misses even with the grouped
-// tile order) and keeps the MFMA pipe 30 % busy.  This kernel doubles the tile both ways, halving
-// the traffic per flop: a workgroup of 8 waves (two per SIMD) owns 256 weight rows x 256
-// activation rows, wave (wm, wn) the 128 activation rows 128 wm .. x the 64 weight rows 64 wn ..
-// (4 x 8 MFMA tiles, 128 fp32 accumulators per lane).  K advances in stages of 64 that go from
-// global memory straight into LDS (global_load_lds_dwordx4: no staging registers, no LDS store
-// instructions), two stage buffers of 64 KiB.  Each load instruction fetches whole 128-byte
-// lines (8 rows x 128 bytes): with stages of 32 (16 rows x 64 bytes per instruction, half lines)
-// the same kernel ran 6-10 % slower, and a timing copy whose loads all hit one L1 line ran 25-30
-// % faster than either -- the cost is in the L1/L2 request stream, not in the LDS writes.  (With
-// the loads staged through registers only one 64-deep stage fitted in flight, and a copy of that
-// kernel without its MFMAs took 539 us of the full kernel's 714 us for a 6144-row gate/up.)
-// SwiGLU: a wave's 64 weight rows are 32 gate rows and the 32 up rows of the same outputs.
-constexpr int BT = 256;                      // weight rows and activation rows per workgroup
-constexpr int BK = 64;                       // K per stage: 128 bytes of every row
-
-// 8 waves (two per SIMD), two along the activation rows and four along the weight rows: wave
-// (wm, wn) owns activation rows 128 wm .. and weight rows 64 wn .. (8 x 4 MFMA tiles, 128 fp32
-// accumulators per lane).  SwiGLU: a wave's 64 weight rows are 32 gate rows and the 32 up rows
-// of the same outputs.  Offsets are 32-bit (checked by the launcher).  (Four waves of 128 x 128,
-// one per SIMD as in hipBLASLt's 256 x 256 tiles, need their 256 accumulators in the AGPRs; with
-// the fragment double buffer below the compiler spilled 241 registers.)
-constexpr int BIG_WAVES = 8;
-template <int EPI>
-__global__ __launch_bounds__(BIG_WAVES * 64, 1) void gemm_big_kernel(
-    const bf16_t* __restrict__ X, int64_t x_stride, int M, const bf16_t* __restrict__ W, int N,
-    int K, int mblocks, int nblocks, bf16_t* out, int64_t out_stride, const bf16_t* res,
-    int64_t res_stride, float* pval, int32_t* pidx, float* logits) {
-  constexpr int WAVES = BIG_WAVES;
-  constexpr int WN = WAVES / 2;              // waves along the weight rows
-  constexpr int NT = BT / WN / 16;           // MFMA tiles per wave along the weight rows
-  constexpr int HALF = NT * 8;               // SwiGLU: gate rows per wave
-  constexpr int ROWS = BT / WAVES;           // LDS rows of each tile a wave loads per stage
-  constexpr int BLK = ROWS / 8;              // ... as 1 KiB blocks of 8 rows (one load each)
-  static_assert(NT == 4 && BLK == 4, "the step below interleaves 4 x 2 loads with 4 x 8 MFMAs");
-  // [stage buffer][weights, activations][row * 8 + position]: row r's 128 bytes hold its eight
-  // 16-byte K units, unit u at position u ^ (r % 8), so that the 8 lanes of a fragment read
-  // (rows c .. c + 7, one unit each) cover all 128 bytes of the banks
-  __shared__ uint4 sm[2][2][BT * 8];
-  const int total = gridDim.x, h = blockIdx.x;
-  const int xq = total >> 3, xr = total & 7, xcd = h & 7, slot = h >> 3;
-  const int L = xcd < xr ? xcd * (xq + 1) + slot : xr * (xq + 1) + (xcd - xr) * xq + slot;
-  const int group = L / (BIG_GROUP_M * nblocks);
-  const int first = group * BIG_GROUP_M;
-  const int gm = min(BIG_GROUP_M, mblocks - first);
-  const int rr = L - first * nblocks;
-  const int mb = first + rr % gm;
-  const int nb = rr / gm;
-
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int c = lane & 15, q = lane >> 4;
-  const int wn = wave % WN, wm = wave / WN;
-  const int64_t m0 = (int64_t)mb * BT;
-  const int stages = K / BK;
-  // weight row of LDS row r: plain nb*256 + r; SwiGLU: LDS rows [2 HALF j, 2 HALF j + HALF) are
-  // the gate rows of outputs nb*128 + HALF j .., the next HALF the up rows (+ N) of the same outputs
-  auto wrow = [&](int r) -> int64_t {
-    if constexpr (EPI == EPI_SWIGLU) {
-      return (int64_t)nb * 128 + HALF * (r / (2 * HALF)) + (r % HALF) + (((r / HALF) & 1) ? N : 0);
-    } else if constexpr (EPI == EPI_ARGMAX) {
-      const int64_t n = (int64_t)nb * BT + r;          // the last block may pass the vocabulary:
-      return n < N ? n : N - 1;                        // reload a valid row, never ranked
-    } else {
-      return (int64_t)nb * BT + r;
-    }
-  };
-  auto xrow = [&](int r) -> int64_t {
-    const int64_t m = m0 + r;
-    return m < M ? m : M - 1;
-  };
-  // loads: wave v fills LDS rows ROWS v .. of both tiles as BLK 1 KiB blocks of 8 rows; lane l
-  // of a block writes position l % 8 of row l / 8 (row % 8 = l / 8), i.e. K unit (l % 8) ^ (l / 8)
-  const int unit = (lane & 7) ^ (lane >> 3);
-  uint32_t wof[BLK], xof[BLK];
-#pragma unroll
-  for (int j = 0; j < BLK; ++j) {
-    const int r = ROWS * wave + 8 * j + (lane >> 3);
-    wof[j] = (uint32_t)(wrow(r) * K * 2 + unit * 16);
-    xof[j] = (uint32_t)(xrow(r) * x_stride * 2 + unit * 16);
-  }
-  const uint32_t lbase = __builtin_amdgcn_readfirstlane(lds_u32(&sm[0][0][0])) + wave * ROWS * 128;
-  constexpr uint32_t XOFF = BT * 8 * 16, BUF = 2 * XOFF;   // activation tile, stage buffer (bytes)
-  // load i (0..7) of stage st into buffer b: weights 0..3, activations 4..7
-  auto load = [&](int st, int b, int i) {
-    const char* base = reinterpret_cast<const char*>(i < BLK ? (const void*)W : (const void*)X) +
-                       (size_t)st * (BK * 2);
-    const int j = i % BLK;
-    dma16(base, i < BLK ? wof[j] : xof[j], lbase + (uint32_t)b * BUF + (i < BLK ? 0u : XOFF) + 1024u * j);
-  };
-  f32x4_t acc[NT][8];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt) acc[nt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // fragment of K half hf (units 4 hf .. 4 hf + 3) of a 16-row tile: lane (c, q) reads unit
-  // 4 hf + q of row tile + c, at position (4 hf + q) ^ (c % 8); tiles are 16 rows = 128 uint4 apart
-  const int pa0 = (64 * wn + c) * 8, pb0 = (128 * wm + c) * 8;
-  const int u0 = q ^ (c & 7), u1 = (4 + q) ^ (c & 7);
-  // fragments of one K half: NT weight tiles, 8 activation tiles (one 16-byte unit per lane each)
-  struct Frag {
-    uint4 a[NT], b[8];
-  };
-  // read fragment t (0..11: weight tiles 0..3, then activation tiles 0..7) of half hf of buffer b
-  auto rd = [&](Frag& f, int b, int hf, int t) {
-    const int u = hf ? u1 : u0;
-    if (t < NT) f.a[t] = sm[b][0][pa0 + 128 * t + u];
-    else f.b[t - NT] = sm[b][1][pb0 + 128 * (t - NT) + u];
-  };
-  // Sub-step j contracts K half j (stage j / 2) from registers while the fragments of half j + 1
-  // are read, in four groups of (two loads, three fragment reads, eight MFMAs) so the load and
-  // LDS instructions issue between MFMAs.  Stage s lives in buffer s % 2.  Odd sub-steps read the
-  // next stage: they first wait for this wave's loads (all of them: stage s + 1 is the only one
-  // in flight) and meet the other waves at a barrier, after which every wave's stage s + 1 has
-  // landed and every wave has read stage s out of its buffer, which then takes stage s + 2 (the
-  // loads of that sub-step).  One barrier per stage.
-  auto sub = [&](int s, int hf, const Frag& cur, Frag& nxt) {
-    const int b = s & 1;
-    const bool ld = hf && s + 2 < stages, rdn = !hf || s + 1 < stages;
-    const int rb = hf ? b ^ 1 : b;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (ld) {
-        load(s + 2, b, 2 * g);
-        load(s + 2, b, 2 * g + 1);
-      }
-      if (rdn) {
-#pragma unroll
-        for (int t = 3 * g; t < 3 * g + 3; ++t) rd(nxt, rb, hf ^ 1, t);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int mt = 2 * g; mt < 2 * g + 2; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-          acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(cur.a[nt]), as_bf8(cur.b[mt]),
-                                                                acc[nt][mt], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-#pragma unroll
-  for (int i = 0; i < 2 * BLK; ++i) load(0, 0, i);
-  if (stages > 1) {
-#pragma unroll
-    for (int i = 0; i < 2 * BLK; ++i) load(1, 1, i);
-    wait_vm<2 * BLK>();                        // stage 0 landed (stage 1 still in flight)
-  } else {
-    wait_vm<0>();
-  }
-  lds_barrier();
-  Frag f0, f1;
-#pragma unroll
-  for (int t = 0; t < NT + 8; ++t) rd(f0, 0, 0, t);
-  for (int s = 0; s < stages; ++s) {
-    sub(s, 0, f0, f1);
-    wait_vm<0>();
-    lds_barrier();
-    sub(s, 1, f1, f0);
-  }
-
-  // epilogue: lane (c, q) of acc[nt][mt] holds weight rows 4 q + r of tile nt = output columns
-  // n .. n + 3 of activation row m = m0 + 128 wm + 16 mt + c
-  if constexpr (EPI == EPI_ARGMAX) {
-    // LM head: per activation row the maximum bf16 logit of the block's 256 vocabulary rows and
-    // its lowest index (the lane's columns ascend with nt and r; lanes and waves hold interleaved
-    // column ranges, so ties compare indices) -> pval / pidx[m][nb] for argmax_reduce_kernel
-    __shared__ float amax_v[2][WN][128];
-    __shared__ int32_t amax_i[2][WN][128];
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt) {
-      const int64_t m = m0 + 128 * wm + 16 * mt + c;
-      float bv = -INFINITY;
-      int32_t bi = 0x7FFFFFFF;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int64_t n = (int64_t)nb * BT + NT * 16 * wn + 16 * nt + 4 * q;
-        if (m < M && logits && n < N)
-          *reinterpret_cast<f32x4_t*>(logits + m * (int64_t)N + n) = acc[nt][mt];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float v = rbf(acc[nt][mt][r]);
-          if (n + r < N && v > bv) { bv = v; bi = (int32_t)(n + r); }
-        }
-      }
-#pragma unroll
-      for (int sh = 0; sh < 2; ++sh) {
-        const float ov = sh ? lane_xor32(bv) : lane_xor16(bv);
-        const int32_t oi = sh ? __builtin_bit_cast(int32_t, lane_xor32(__builtin_bit_cast(float, bi)))
-                              : __builtin_bit_cast(int32_t, lane_xor16(__builtin_bit_cast(float, bi)));
-        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-      }
-      if (q == 0) {
-        amax_v[wm][wn][16 * mt + c] = bv;
-        amax_i[wm][wn][16 * mt + c] = bi;
-      }
-    }
-    lds_barrier();
-    if (tid < 256) {
-      const int wm2 = tid >> 7, r = tid & 127;
-      const int64_t m = m0 + 128 * wm2 + r;
-      if (m < M) {
-        float bv = amax_v[wm2][0][r];
-        int32_t bi = amax_i[wm2][0][r];
-#pragma unroll
-        for (int w = 1; w < WN; ++w) {
-          const float ov = amax_v[wm2][w][r];
-          const int32_t oi = amax_i[wm2][w][r];
-          if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-        }
-        pval[m * (int64_t)nblocks + nb] = bv;
-        pidx[m * (int64_t)nblocks + nb] = bi;
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int mt = 0; mt < 8; ++mt) {
-    const int64_t m = m0 + 128 * wm + 16 * mt + c;
-    if (m >= M) continue;
-    if constexpr (EPI == EPI_SWIGLU) {
-#pragma unroll
-      for (int nt = 0; nt < NT / 2; ++nt) {
-        const int64_t n = (int64_t)nb * 128 + HALF * wn + 16 * nt + 4 * q;
-        float y[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          y[r] = silu_rbf(rbf(acc[nt][mt][r])) * rbf(acc[nt + NT / 2][mt][r]);
-        *reinterpret_cast<uint2*>(out + m * out_stride + n) = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-      }
-    } else {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int64_t n = (int64_t)nb * BT + NT * 16 * wn + 16 * nt + 4 * q;
-        float y[4];
-        if constexpr (EPI == EPI_RES) {
-          const uint2 rv = *reinterpret_cast<const uint2*>(res + m * res_stride + n);
-          y[0] = bflo(rv.x) + rbf(acc[nt][mt][0]);
-          y[1] = bfhi(rv.x) + rbf(acc[nt][mt][1]);
-          y[2] = bflo(rv.y) + rbf(acc[nt][mt][2]);
-          y[3] = bfhi(rv.y) + rbf(acc[nt][mt][3]);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) y[r] = acc[nt][mt][r];
-        }
-        *reinterpret_cast<uint2*>(out + m * out_stride + n) = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-      }
-    }
-  }
 }
 
 // ------------------------------------------------------------------ all rows per workgroup (65..256)
@@ -1153,15 +730,12 @@ int gemm_tile_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
   const int ksteps = (int)(K / TK);
   const int ks_per = (ksteps + splits - 1) / splits;
   splits = (ksteps + ks_per - 1) / ks_per;              // no empty split
+  if (launch_gemm_quad(x, xs, M, w, N, K, nullptr, 0, nullptr, 0, EPI_NONE, splits, ks_per, part, s))
+    return splits;
   const int64_t mblocks = (M + TM - 1) / TM, nblocks = tile_nblocks(N, EPI_NONE);
-  if (QD_TILE8)
-    gemm_tile8_kernel<EPI_NONE, true><<<dim3((unsigned)(mblocks * nblocks * splits)), dim3(512), 0, s>>>(
-        x, xs, (int)M, w, (int)N, (int)K, (int)mblocks, (int)nblocks, ks_per, nullptr, 0, nullptr,
-        0, part);
-  else
-    gemm_tile_kernel<EPI_NONE, true><<<dim3((unsigned)(mblocks * nblocks * splits)), dim3(256), 0, s>>>(
-        x, xs, (int)M, w, (int)N, (int)K, (int)mblocks, (int)nblocks, ks_per, nullptr, 0, nullptr,
-        0, nullptr, nullptr, nullptr, part);
+  gemm_tile_kernel<EPI_NONE, true><<<dim3((unsigned)(mblocks * nblocks * splits)), dim3(256), 0, s>>>(
+      x, xs, (int)M, w, (int)N, (int)K, (int)mblocks, (int)nblocks, ks_per, nullptr, 0, nullptr, 0,
+      nullptr, nullptr, nullptr, part);
   return splits;
 }
 
@@ -1170,29 +744,9 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
                          int64_t K, bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi,
                          float* pval, int32_t* pidx, float* logits, float* part,
                          int64_t part_floats, hipStream_t s) {
-  if (epi != EPI_ARGMAX && ((QD_BIG_EPIS >> epi) & 1) && M >= QD_BIG_MIN_M &&
-      (epi == EPI_SWIGLU ? N % 128 == 0 : N % BT == 0) &&
-      (epi == EPI_SWIGLU ? 2 * N : N) * K * 2 < (1ll << 32) && M * xs * 2 < (1ll << 32)) {
-    const int64_t mbl = (M + BT - 1) / BT, nbl = epi == EPI_SWIGLU ? N / 128 : N / BT;
-    const dim3 g((unsigned)(mbl * nbl)), b(BIG_WAVES * 64);
-#define QD_BIG(E) \
-  gemm_big_kernel<E><<<g, b, 0, s>>>(x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, out, os, res, rs, \
-                                     nullptr, nullptr, nullptr)
-    if (epi == EPI_RES) QD_BIG(EPI_RES);
-    else if (epi == EPI_SWIGLU) QD_BIG(EPI_SWIGLU);
-    else QD_BIG(EPI_NONE);
-#undef QD_BIG
-    return 0;
-  }
-  if (epi == EPI_ARGMAX && M >= QD_BIG_ARGMAX_MIN_M && N % 4 == 0 && N >= BT &&
-      N * K * 2 < (1ll << 32) && M * xs * 2 < (1ll << 32)) {
-    // LM head over many rows (a tree verification's 256): 256 x 256 tiles read every weight
-    // byte once per 256 activation rows, half the L2 traffic of the 128 x 128 tiles
-    const int64_t mbl = (M + BT - 1) / BT, nbl = (N + BT - 1) / BT;
-    gemm_big_kernel<EPI_ARGMAX><<<dim3((unsigned)(mbl * nbl)), dim3(BIG_WAVES * 64), 0, s>>>(
-        x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, nullptr, 0, nullptr, 0, pval, pidx,
-        logits);
-    return nbl;
+  if (epi == EPI_ARGMAX) {
+    const int64_t parts = launch_lm_quad(x, xs, M, w, N, K, pval, pidx, logits, s);
+    if (parts > 0) return parts;
   }
   RowsPlan P;
   if (epi != EPI_ARGMAX && rows_launch_plan(M, N, K, epi, false, part ? part_floats : 0, P) == 1) {
@@ -1216,19 +770,21 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
     return 0;
   }
   const int64_t mblocks = (M + TM - 1) / TM, nblocks = tile_nblocks(N, epi);
-  int splits = gemm_tile_splits(M, N, K, epi);
+  // from 1024 rows on, whole 256-column blocks are not split (the largest tiles fill the chip)
+  int splits = M >= 1024 && N % 256 == 0 ? 1 : gemm_tile_splits(M, N, K, epi);
   if (splits > 1 && (!part || part_floats < (int64_t)splits * M * N)) splits = 1;
   const int ksteps = (int)(K / TK);
   const int ks_per = (ksteps + splits - 1) / splits;
   splits = (ksteps + ks_per - 1) / ks_per;              // no empty split
+  // the four-wave kernel; the 128 x 128 tiles below where its 32-bit offsets do not reach, and
+  // for the LM head's 65..128 rows
+  const bool quad = epi != EPI_ARGMAX &&
+                    launch_gemm_quad(x, xs, M, w, N, K, out, os, res, rs, epi, splits, ks_per, part, s);
   const dim3 grid((unsigned)(mblocks * nblocks * splits)), block(256);
   const int Mi = (int)M, Ni = (int)N, Ki = (int)K, mbi = (int)mblocks, nbi = (int)nblocks;
 #define QD_TILE(E, SP)                                                                           \
   do {                                                                                           \
-    if (QD_TILE8 && E != EPI_ARGMAX)                                                             \
-      gemm_tile8_kernel<E == EPI_ARGMAX ? EPI_NONE : E, SP><<<grid, dim3(512), 0, s>>>(          \
-          x, xs, Mi, w, Ni, Ki, mbi, nbi, ks_per, out, os, res, rs, part);                       \
-    else                                                                                         \
+    if (!quad)                                                                                   \
       gemm_tile_kernel<E, SP><<<grid, block, 0, s>>>(x, xs, Mi, w, Ni, Ki, mbi, nbi, ks_per, out, \
                                                      os, res, rs, pval, pidx, logits, part);     \
   } while (0)

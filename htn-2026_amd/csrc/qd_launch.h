@@ -97,6 +97,12 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
                          int64_t K, bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi,
                          float* pval, int32_t* pidx, float* logits, float* part,
                          int64_t part_floats, hipStream_t s);
+// gemm_quad.hip (four-wave MFMA GEMM, 257 and more rows; the LM head from 129 rows)
+bool launch_gemm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
+                      bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi, int splits,
+                      int ks_per, float* part, hipStream_t s);
+int64_t launch_lm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
+                       float* pval, int32_t* pidx, float* logits, hipStream_t s);
 // rows from which the tiled kernel takes over
 constexpr int64_t GEMM_TILE_MIN_M = 65;
 

@@ -1,0 +1,95 @@
+"""The four-wave GEMM of 257 and more rows (gemm_quad.hip): every tile shape its plan picks for the
+model's projections, ragged row counts around the tiles, and outputs that are only 8-byte aligned.
+
+An output's accumulation runs through K in order whatever the tile, so unsplit launches agree bit
+for bit on the rows they share; the largest launch is held to an fp64 product."""
+
+import pytest
+import torch
+
+from helpers import bf16_ulp
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+SHAPES = {"qkv": (6144, 2560), "o": (2560, 4096), "gu": (9728, 2560), "down": (2560, 9728)}
+# between them these counts take all 13 tile shapes; 257, 1025 and 2049 leave one row in the last
+# row block, 1023 and 4095 fill all but one
+ROWS = [257, 300, 399, 513, 601, 768, 1023, 1025, 1500, 2049, 3000, 4095, 6001]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from qdecode import ops as o
+    return o
+
+
+def _operands(name, M):
+    N, K = SHAPES[name]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K)
+    r = lambda *s, std=1.0: torch.empty(s, dtype=BF, device="cuda").normal_(0, std, generator=g)  # noqa: E731
+    return r(M, K), r(2 * N if name == "gu" else N, K, std=0.02), r(M, N, std=2.0)
+
+
+def _linear(ops, name, x, w, res, **kw):
+    epi = {"qkv": ops.EPI_NONE, "gu": ops.EPI_SWIGLU}.get(name, ops.EPI_RES)
+    return ops.linear(x, w, epi, res=res[:x.shape[0]] if epi == ops.EPI_RES else None, **kw)
+
+
+@pytest.mark.parametrize("name", list(SHAPES))
+def test_every_tile_shape_agrees(ops, name):
+    N, K = SHAPES[name]
+    x, w, res = _operands(name, ROWS[-1])
+    print(f"\n[case] {name}: {ROWS} rows", flush=True)
+    full = _linear(ops, name, x, w, res)
+    acc = x.double() @ w.double().t()
+    if name == "gu":
+        # first-order propagation of one ulp in bf16(gate), bf16(up) and bf16(silu), two of output
+        gate, up = acc[:, :N].to(BF).float(), acc[:, N:].to(BF).float()
+        sg = torch.sigmoid(gate)
+        s = (gate * sg).to(BF).float()
+        want = (s * up).to(BF)
+        dsilu = (sg * (1 + gate * (1 - sg))).abs()
+        bound = (up.abs() * (dsilu * bf16_ulp(gate) + bf16_ulp(s)) + s.abs() * bf16_ulp(up)
+                 + 2 * bf16_ulp(torch.maximum(full.float().abs(), want.float().abs())) + 2 ** -12)
+    elif name == "qkv":
+        want = acc.to(BF)
+        bound = 2 * bf16_ulp(torch.maximum(full.float().abs(), want.float().abs())) + 2 ** -9
+    else:
+        a = acc.to(BF).float()
+        want = (res.float() + a).to(BF)
+        bound = bf16_ulp(a) + 2 * bf16_ulp(torch.maximum(full.float().abs(), want.float().abs()))
+    d = (full.float() - want.float()).abs()
+    assert bool((d <= bound).all()), f"max excess {float((d - bound).max())}"
+    for M in ROWS[:-1]:
+        if name in ("o", "down") and M < 1024:
+            continue                             # K is split: other sums (tested with the splits)
+        part = _linear(ops, name, x[:M], w, res)
+        assert torch.equal(part.view(torch.int16), full[:M].view(torch.int16)), f"{M} rows"
+
+
+@pytest.mark.parametrize("name", ["o", "down"])
+@pytest.mark.parametrize("M", [257, 384, 513, 1023])
+def test_split_launches(ops, name, M):
+    x, w, res = _operands(name, M)
+    got = _linear(ops, name, x, w, res).float()
+    a = (x.double() @ w.double().t()).to(BF).float()
+    want = (res.float() + a).to(BF).float()
+    bound = bf16_ulp(a) + 2 * bf16_ulp(torch.maximum(got.abs(), want.abs()))
+    assert bool(((got - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("name,M", [("qkv", 300), ("gu", 601), ("down", 1500), ("o", 4095)])
+def test_outputs_aligned_to_8_bytes(ops, name, M):
+    """An output (and residual) whose rows start 8 bytes off a 16-byte boundary takes the narrow
+    stores: the same bits, and nothing written beside the rows."""
+    x, w, res = _operands(name, M)
+    N = SHAPES[name][0]
+    want = _linear(ops, name, x, w, res)
+    buf = torch.full((M, N + 12), 7.0, dtype=BF, device="cuda")
+    rbuf = torch.zeros((M, N + 12), dtype=BF, device="cuda")
+    out, r2 = buf[:, 4:4 + N], rbuf[:, 4:4 + N]
+    r2.copy_(res)
+    _linear(ops, name, x, w, r2, out=out)
+    assert torch.equal(out, want)
+    assert bool((buf[:, :4] == 7).all()) and bool((buf[:, 4 + N:] == 7).all())
