@@ -284,10 +284,10 @@ void launch_part_add_rmsnorm(const float* part, int S, int64_t rows, bf16_t* res
   const dim3 g((unsigned)rows), b(256);
   if (hidden / 8 > 256 && hidden / 8 <= 512) {
     switch (S) {
-      case 1: part_add_rmsnorm2_kernel<1><<<g, b, 0, s>>>(part, rows, res, w, y, hidden, eps); return;
-      case 2: part_add_rmsnorm2_kernel<2><<<g, b, 0, s>>>(part, rows, res, w, y, hidden, eps); return;
-      case 4: part_add_rmsnorm2_kernel<4><<<g, b, 0, s>>>(part, rows, res, w, y, hidden, eps); return;
-      case 6: part_add_rmsnorm2_kernel<6><<<g, b, 0, s>>>(part, rows, res, w, y, hidden, eps); return;
+#define QD_PAR(SC)                                                                             \
+  case SC: part_add_rmsnorm2_kernel<SC><<<g, b, 0, s>>>(part, rows, res, w, y, hidden, eps); return
+      QD_PAR(1); QD_PAR(2); QD_PAR(3); QD_PAR(4); QD_PAR(5); QD_PAR(6); QD_PAR(7); QD_PAR(8);
+#undef QD_PAR
       default: break;
     }
   }

@@ -577,19 +577,24 @@ static int64_t gemm_mt(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
                        int64_t K, bf16_t* out, int64_t os, const bf16_t* res, int64_t rs,
                        float* pval, int32_t* pidx, float* logits, float* part, int64_t part_floats,
                        hipStream_t s) {
-  if (M >= GEMM_TILE_MIN_M && gemm_tile_ok(M, N, K, EPI, x, xs, w, out, os, res, rs))
+  if (M >= (EPI == EPI_ARGMAX ? GEMM_TILE_MIN_M : GEMM_SMALL_MIN_M) &&
+      gemm_tile_ok(M, N, K, EPI, x, xs, w, out, os, res, rs))
     return launch_gemm_tile(x, xs, M, w, N, K, out, os, res, rs, EPI, pval, pidx, logits, part,
                             part_floats, s);
   const int P = stream_grid();
   const bool aligned = xs % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(w) % 16 == 0;
   // the LM head: 3..32 rows on the skinny argmax kernel (activations resident in LDS per K
-  // phase); 33..64 rows on the weight-streaming kernel (~600 rows per workgroup, so its per-chunk
-  // activation re-reads stay small next to the weight rows); the projections: 3..32 rows on the
-  // skinny kernel, 33..64 on the LDS-staged one
+  // phase); 33..64 rows on the four-wave kernel; the projections: 3..32 rows on the skinny kernel,
+  // 33..64 on the four-wave one.  What those do not take (unaligned operands, odd widths): the
+  // weight-streaming and LDS-staged kernels here
   if constexpr (EPI == EPI_ARGMAX) {
     if (M <= 32) {
       const int64_t parts = launch_lm_skinny(x, xs, M, w, N, K, pval, pidx, logits, s);
+      if (parts > 0) return parts;
+    }
+    if (M > 32 && M <= 64) {
+      const int64_t parts = launch_lm_quad(x, xs, M, w, N, K, pval, pidx, logits, s);
       if (parts > 0) return parts;
     }
     if (M <= 64 && K % 512 == 0 && aligned && P >= 1) {

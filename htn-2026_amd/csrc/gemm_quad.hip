@@ -61,15 +61,17 @@ __host__ __device__ constexpr int quad_lds_u4(int mt, int nt, int nbuf) {
   return nbuf * 32 * (mt + nt) * 8 + (nbuf == 2 ? 16 : 0);   // stages, and the touched dwords
 }
 
+// output columns of a workgroup's tile
+__host__ __device__ constexpr int quad_outs(int nt, bool sw) { return sw ? 16 * nt : 32 * nt; }
+
 template <int EPI, bool SPLIT, int MT, int NT, int NBUF>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
     const bf16_t* __restrict__ X, int64_t x_stride, int M, const bf16_t* __restrict__ W, int N,
-    int K, int mblocks, int nblocks, int ks_per, bf16_t* out, int64_t out_stride,
+    int K, int mblocks, int nblocks, int outs, int ks_per, bf16_t* out, int64_t out_stride,
     const bf16_t* res, int64_t res_stride, int wide, float* part, float* pval, int32_t* pidx,
     float* logits) {
   constexpr bool SW = EPI == EPI_SWIGLU && !SPLIT;
   constexpr int BM = 32 * MT, BN = 32 * NT, ROWS = BM + BN;   // LDS rows: weights, activations
-  constexpr int OUTS = SW ? BN / 2 : BN;       // output columns per workgroup
   constexpr int PER = MT + NT;                 // 1 KiB load blocks per wave and stage
   constexpr int GT = SW ? NT / 2 : NT;         // tiles of one run of weight rows (gate, up)
   constexpr int PAIRED = 32 * (GT / 2);        // its interleaved rows; an odd last tile follows
@@ -95,8 +97,8 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
   const int c = lane & 15, q = lane >> 4;
   const int wn = wave & 1, wm = wave >> 1;
   const int64_t m0 = (int64_t)mb * BM;
-  const int n0 = nb * OUTS;
-  const int nrows = min(OUTS, N - n0);
+  const int n0 = nb * outs;                    // output columns per workgroup: at most quad_outs()
+  const int nrows = min(outs, N - n0);
   const int mrows = (int)(M - m0 < BM ? M - m0 : BM);
   const int kbeg = split * ks_per;
   const int stages = min(K / TK, kbeg + ks_per) - kbeg;
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
       const bool paired = 32 * (i / 2) < PAIRED;
       if (paired && (i & 1)) continue;         // with its even tile
       const int u = 16 * GT * wn + (paired ? 16 * i + 8 * q : 16 * i + 4 * q);
-      if (u >= nrows) continue;                // N and the blocks are multiples of 32 columns
+      if (u >= nrows) continue;                // N and outs are multiples of 8 columns
       const int64_t n = (int64_t)n0 + u;
       {
         const f32x4_t lo = acc[i][mt], hi = acc[paired ? i + 1 : i][mt];
@@ -390,7 +392,7 @@ int quad_plan(int64_t M, int64_t N, bool sw, int64_t splits, int64_t stages) {
   for (int i = 0; i < QUADS; ++i) {
     const QuadShape& q = QUAD[i];
     if (sw && q.nt % 2) continue;
-    const int64_t bm = 32 * q.mt, bn = sw ? 16 * q.nt : 32 * q.nt;
+    const int64_t bm = 32 * q.mt, bn = quad_outs(q.nt, sw);
     const int64_t wgs = (M + bm - 1) / bm * ((N + bn - 1) / bn) * splits;
     const double t = (double)((wgs + quad_cus() - 1) / quad_cus()) *
                      (q.a + (sw ? QUAD_SWIGLU * q.mt * q.nt : 0.0) + (double)q.b * stages);
@@ -407,10 +409,10 @@ void quad_go(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,
              int64_t os, const bf16_t* res, int64_t rs, int splits, int ks_per, int wide,
              float* part, hipStream_t s) {
   constexpr QuadShape q = QUAD[I];
-  constexpr int BM = 32 * q.mt, BN = EPI == EPI_SWIGLU ? 16 * q.nt : 32 * q.nt;
+  constexpr int BM = 32 * q.mt, BN = quad_outs(q.nt, EPI == EPI_SWIGLU);
   const int64_t mbl = (M + BM - 1) / BM, nbl = (N + BN - 1) / BN;
   gemm_quad_kernel<EPI, SPLIT, q.mt, q.nt, q.nbuf><<<dim3((unsigned)(mbl * nbl * splits)), dim3(256), 0, s>>>(
-      x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, ks_per, out, os, res, rs, wide, part,
+      x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, BN, ks_per, out, os, res, rs, wide, part,
       nullptr, nullptr, nullptr);
 }
 
@@ -455,16 +457,130 @@ bool launch_gemm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, i
   return true;
 }
 
-// LM head over 129 and more rows: argmax partials pval / pidx [M][return value] (256 vocabulary
-// rows each; the last block may pass the vocabulary: its missing rows reload a valid one and are
-// never ranked); 0, with nothing launched, for other shapes.  (256 rows, one row block: 594
-// workgroups of 256 x 256.)
+// ------------------------------------------------------------------ 33..64 rows
+// A batched decode step or a small tree: every weight byte is used 64 times at most and read once,
+// so the weight stream is the cost and the workgroups (one row block of 64) must take equal shares
+// of it in one round.  (Also the split partials of a decode step of 65..128 rows, two row blocks:
+// its room for partials holds fewer splits than the all-rows kernel's plan there takes.)  Shapes
+// {2, NT}; outs <= quad_outs(NT) columns per workgroup and S K splits
+// (fp32 partials, for the store / residual products), the pair that costs least:
+//   2.5 us + (0.08 + 0.0027 weight rows + 0.0018 staged weight rows) us per stage
+//   + 8 S M N bytes of partials written and read back at 4 TB/s,
+// fitted on MI355X to shapes {2, 2} .. {2, 6} and 1 to 8 splits at 33, 48 and 64 rows.  At 48 rows
+// (weights from HBM, partials not reduced): qkv 20.8 -> 9.2 us, o 18.4 -> 6.3, gate/up 48.7 ->
+// 28.3, down 36.3 -> 11.8 against the 16-row weight tiles of gemm_lds_kernel, which read every
+// weight twice above 32 rows (reading the weights alone: 4.8, 3.2, 15.3, 7.7 us).
+struct SmallPlan {
+  int nt = 0, outs = 0, splits = 1, ks_per = 0;
+};
+constexpr int SMALL_SPLITS = 8;
+
+static SmallPlan quad_small_plan(int64_t M, int64_t N, int64_t K, bool sw, int64_t max_splits) {
+  SmallPlan best;
+  double best_t = 0;
+  const int64_t stages = K / TK, mbl = (M + 63) / 64;
+  if (max_splits > SMALL_SPLITS) max_splits = SMALL_SPLITS;
+  if (sw || max_splits < 1) max_splits = 1;
+  for (int64_t S0 = 1; S0 <= max_splits && (S0 == 1 || stages / S0 >= 4); ++S0) {
+    const int64_t ks_per = (stages + S0 - 1) / S0, S = (stages + ks_per - 1) / ks_per;
+    for (int nt = 2; nt <= 6; ++nt) {
+      if (nt == 5 || (sw && nt % 2)) continue;
+      const int64_t most = quad_outs(nt, sw);
+      const int64_t blocks = quad_cus() / (S * mbl) > 0 ? quad_cus() / (S * mbl) : 1;   // one round
+      int64_t outs = ((N + blocks - 1) / blocks + 7) / 8 * 8;
+      if (outs > most) outs = most;
+      const int64_t wgs = (N + outs - 1) / outs * S * mbl;
+      const double rows = (double)outs * (sw ? 2 : 1);
+      const double t = (double)((wgs + quad_cus() - 1) / quad_cus()) *
+                           (2.5 + (0.08 + 0.0027 * rows + 0.0018 * 32 * nt) * (double)ks_per) +
+                       (S > 1 ? 8.0 * S * M * N / 4e6 : 0.0);
+      if (best.nt == 0 || t < best_t) {
+        best_t = t;
+        best.nt = nt;
+        best.outs = (int)outs;
+        best.splits = (int)S;
+        best.ks_per = (int)ks_per;
+      }
+    }
+  }
+  return best;
+}
+
+template <int EPI, bool SPLIT>
+static void quad_small_go(const SmallPlan& P, const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w,
+                          int64_t N, int64_t K, bf16_t* out, int64_t os, const bf16_t* res,
+                          int64_t rs, int wide, float* part, hipStream_t s) {
+  const int64_t mbl = (M + 63) / 64, nbl = (N + P.outs - 1) / P.outs;
+#define QD_SMALL(NT, NB)                                                                        \
+  gemm_quad_kernel<EPI, SPLIT, 2, NT, NB><<<dim3((unsigned)(mbl * nbl * P.splits)), dim3(256), 0, s>>>( \
+      x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, P.outs, P.ks_per, out, os, res, rs, wide, part, \
+      nullptr, nullptr, nullptr)
+  if (P.nt == 2) QD_SMALL(2, 4);
+  else if (P.nt == 4) QD_SMALL(4, 3);
+  else if (P.nt == 6) QD_SMALL(6, 4);
+  else if constexpr (EPI != EPI_SWIGLU) QD_SMALL(3, 3);
+#undef QD_SMALL
+}
+
+// The operands satisfy gemm_tile_ok, 33 <= M <= 64 (quad_small_partials: 128).  quad_small_partials: fp32 partials
+// part[S][M][N], S returned (0, nothing launched: no split fits part_floats or pays).
+// launch_quad_small: the whole product; with splits its partials go to part, their count is
+// returned and the caller reduces them, else 0 is returned and out is written; -1, with nothing
+// launched, where the 32-bit offsets do not reach.
+int quad_small_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
+                        float* part, int64_t part_floats, hipStream_t s) {
+  if (!quad_offsets_ok(xs, N, K, EPI_NONE)) return 0;
+  const SmallPlan P = quad_small_plan(M, N, K, false, part ? part_floats / (M * N) : 1);
+  if (P.splits <= 1) return 0;
+  quad_small_go<EPI_NONE, true>(P, x, xs, M, w, N, K, nullptr, 0, nullptr, 0, 0, part, s);
+  return P.splits;
+}
+
+int launch_quad_small(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
+                      bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi, float* part,
+                      int64_t part_floats, hipStream_t s) {
+  if (!quad_offsets_ok(xs, N, K, epi)) return -1;
+  const SmallPlan P = quad_small_plan(M, N, K, epi == EPI_SWIGLU, part ? part_floats / (M * N) : 1);
+  const int wide = (al16(out, os) ? 1 : 0) | (res && al16(res, rs) ? 2 : 0);
+  if (P.splits > 1) {
+    quad_small_go<EPI_NONE, true>(P, x, xs, M, w, N, K, nullptr, 0, nullptr, 0, 0, part, s);
+    return P.splits;
+  }
+  if (epi == EPI_RES) quad_small_go<EPI_RES, false>(P, x, xs, M, w, N, K, out, os, res, rs, wide, part, s);
+  else if (epi == EPI_SWIGLU) quad_small_go<EPI_SWIGLU, false>(P, x, xs, M, w, N, K, out, os, res, rs, wide, part, s);
+  else quad_small_go<EPI_NONE, false>(P, x, xs, M, w, N, K, out, os, res, rs, wide, part, s);
+  return 0;
+}
+
+// split partials the two above can use at most
+int64_t quad_small_ws_floats(int64_t M, int64_t N, int64_t K) {
+  const SmallPlan P = quad_small_plan(M, N, K, false, SMALL_SPLITS);
+  return P.splits > 1 ? (int64_t)P.splits * M * N : 0;
+}
+
+// LM head over 33..64 and 129 and more rows: argmax partials pval / pidx [M][return value] (one per
+// block of vocabulary rows; the last block may pass the vocabulary: its missing rows reload a valid
+// one and are never ranked); 0, with nothing launched, for other shapes.  129 and more rows: 256 x
+// 256 tiles.  33..64 rows: 320 vocabulary rows per workgroup, two nearly full rounds (475
+// workgroups at 151936), 64 KiB of weights in flight per CU: 40 rows 275 -> 138 us (5.6 TB/s) against
+// gemm_stream_kernel, which re-stages the activations with every chunk; 64 rows 285 -> 139 us
+// ({2, 4} tiles 139 / 146, {2, 8} 157 / 159).  65..128 rows stay on gemm_tile_kernel: 167 us at
+// 100 rows against 174 with {4, 8} tiles here.
 int64_t launch_lm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
                        float* pval, int32_t* pidx, float* logits, hipStream_t s) {
-  if (M < 129 || M >= (1ll << 31) || N % 4 || N < 256 || !quad_offsets_ok(xs, N, K, EPI_ARGMAX)) return 0;
-  const int64_t mbl = (M + 255) / 256, nbl = (N + 255) / 256;
-  gemm_quad_kernel<EPI_ARGMAX, false, 8, 8, 2><<<dim3((unsigned)(mbl * nbl)), dim3(256), 0, s>>>(
-      x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, (int)(K / TK), nullptr, 0, nullptr, 0, 0,
-      nullptr, pval, pidx, logits);
+  const bool small = M >= 33 && M <= 64;
+  if ((!small && M < 129) || M >= (1ll << 31) || N % 4 || N < 256 || K % TK ||
+      !quad_offsets_ok(xs, N, K, EPI_ARGMAX))
+    return 0;
+  if (xs % 8 || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16) return 0;
+  const int64_t bm = small ? 64 : 256, bn = small ? 320 : 256;
+  const int64_t mbl = (M + bm - 1) / bm, nbl = (N + bn - 1) / bn;
+#define QD_LM(MT, NT, NB)                                                                       \
+  gemm_quad_kernel<EPI_ARGMAX, false, MT, NT, NB><<<dim3((unsigned)(mbl * nbl)), dim3(256), 0, s>>>( \
+      x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, (int)bn, (int)(K / TK), nullptr, 0, nullptr, \
+      0, 0, nullptr, pval, pidx, logits)
+  if (small) QD_LM(2, 10, 3);
+  else QD_LM(8, 8, 2);
+#undef QD_LM
   return nbl;
 }

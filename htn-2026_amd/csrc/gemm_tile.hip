@@ -707,16 +707,28 @@ int gemm_rows_query(int64_t M, int64_t N, int64_t K, int epi, bool partials_only
 }
 
 int64_t gemm_tile_ws_floats(int64_t M, int64_t N, int64_t K, int epi) {
+  if (M < GEMM_TILE_MIN_M) return M >= GEMM_SMALL_MIN_M && K % TK == 0 ? quad_small_ws_floats(M, N, K) : 0;
   RowsPlan P;
   const int sp = rows_plan(M, N, K, epi, true, P) ? P.splits : gemm_tile_splits(M, N, K, epi);
   return sp > 1 ? (int64_t)sp * M * N : 0;
 }
 
+// as gemm_tile_partials, for a decode step's rows: where the all-rows kernel's split count does
+// not fit part_floats, the four-wave kernel takes fewer
+int gemm_step_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,
+                       int64_t K, float* part, int64_t part_floats, hipStream_t s) {
+  if (M > 128 || gemm_tile_ws_floats(M, N, K, EPI_NONE) <= part_floats)
+    return gemm_tile_partials(x, xs, M, w, N, K, part, part_floats, s);
+  if (M < GEMM_SMALL_MIN_M || !gemm_tile_ok(M, N, K, EPI_NONE, x, xs, w, part, N, nullptr, 0)) return 0;
+  return quad_small_partials(x, xs, M, w, N, K, part, part_floats, s);
+}
+
 int gemm_tile_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,
                        int64_t K, float* part, int64_t part_floats, hipStream_t s) {
-  if (M < GEMM_TILE_MIN_M || !part ||
+  if (M < GEMM_SMALL_MIN_M || !part ||
       !gemm_tile_ok(M, N, K, EPI_NONE, x, xs, w, part, N, nullptr, 0))
     return 0;
+  if (M < GEMM_TILE_MIN_M) return quad_small_partials(x, xs, M, w, N, K, part, part_floats, s);
   RowsPlan P;
   const int rp = rows_launch_plan(M, N, K, EPI_NONE, true, part_floats, P);
   if (rp == 0) return 0;
@@ -748,17 +760,24 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
     const int64_t parts = launch_lm_quad(x, xs, M, w, N, K, pval, pidx, logits, s);
     if (parts > 0) return parts;
   }
+  auto reduce = [&](int S) {
+    const dim3 rg((unsigned)((M * (N / 4) + 255) / 256)), rb(256);
+    if (epi == EPI_RES)
+      gemm_split_reduce_kernel<EPI_RES><<<rg, rb, 0, s>>>(part, S, M, N, out, os, res, rs);
+    else
+      gemm_split_reduce_kernel<EPI_NONE><<<rg, rb, 0, s>>>(part, S, M, N, out, os, res, rs);
+  };
+  if (epi != EPI_ARGMAX && M < GEMM_TILE_MIN_M) {
+    const int S = launch_quad_small(x, xs, M, w, N, K, out, os, res, rs, epi, part, part ? part_floats : 0, s);
+    if (S > 0) reduce(S);
+    if (S >= 0) return 0;
+  }
   RowsPlan P;
   if (epi != EPI_ARGMAX && rows_launch_plan(M, N, K, epi, false, part ? part_floats : 0, P) == 1) {
     if (P.splits > 1) {
       launch_rows<EPI_NONE, true>(P, x, xs, (int)M, w, (int)N, (int)K, nullptr, 0, nullptr, 0,
                                   part, s);
-      const int64_t thr = M * (N / 4);
-      const dim3 rg((unsigned)((thr + 255) / 256)), rb(256);
-      if (epi == EPI_RES)
-        gemm_split_reduce_kernel<EPI_RES><<<rg, rb, 0, s>>>(part, P.splits, M, N, out, os, res, rs);
-      else
-        gemm_split_reduce_kernel<EPI_NONE><<<rg, rb, 0, s>>>(part, P.splits, M, N, out, os, res, rs);
+      reduce(P.splits);
       return 0;
     }
     if (epi == EPI_RES)
@@ -791,12 +810,7 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
   if (splits > 1) {
     if (epi == EPI_RES) QD_TILE(EPI_RES, true);
     else QD_TILE(EPI_NONE, true);
-    const int64_t thr = M * (N / 4);
-    const dim3 rg((unsigned)((thr + 255) / 256));
-    if (epi == EPI_RES)
-      gemm_split_reduce_kernel<EPI_RES><<<rg, block, 0, s>>>(part, splits, M, N, out, os, res, rs);
-    else
-      gemm_split_reduce_kernel<EPI_NONE><<<rg, block, 0, s>>>(part, splits, M, N, out, os, res, rs);
+    reduce(splits);
     return 0;
   }
   switch (epi) {

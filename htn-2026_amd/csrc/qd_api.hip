@@ -435,6 +435,55 @@ int qd_decode_step(const qd_weights* w, const qd_decode_state* st, void* stream)
     launch_part_add_rmsnorm(part, SK_SPLIT_DOWN, B, st->x, w->final_norm, lw.xn, H, w->eps, s);
     return lm_head_normed(lw.xn, lm_weight(w), V, H, B, st->tok, st->pos, lw, s);
   }
+  if (B > 32) {
+    // 33 rows and more: the qkv, o and down projections leave K-split partials where their plan
+    // splits, summed by the attention prologue and the next residual add + RMSNorm (as the block
+    // step does).  They sit in the LM head's partial region (val and idx, adjacent), which is idle
+    // until the last layer's have been summed, so the step needs no more workspace than before;
+    // a projection whose partials do not fit takes fewer splits, or none.  Step times, unsplit
+    // projections before -> now (MI355X): 48 rows, 36 layers, context 1500 7.44 -> 5.00 ms; 4
+    // layers: 36 rows, context 1000 1283 -> 752 us, 70 rows, context 300 1042 -> 824, 128 rows
+    // 1162 -> 959.
+    float* part = lw.val;
+    const int64_t room = (reinterpret_cast<char*>(lw.xn) - reinterpret_cast<char*>(lw.val)) / 4;
+    int pend = 0;                                // splits of down partials not yet in x
+    for (int64_t l = 0; l < w->n_layers; ++l) {
+      const bf16_t *wqkv = w->w_qkv + l * NQKV * H, *wo = w->w_o + l * H * QD;
+      const bf16_t *wgu = w->w_gu + l * 2 * I * H, *wd = w->w_down + l * H * I;
+      bf16_t *kc = st->k_cache + l * layer_kv, *vc = st->v_cache + l * layer_kv;
+      if (pend) launch_part_add_rmsnorm(part, pend, B, st->x, w->ln1 + l * H, xn, H, w->eps, s);
+      else launch_add_rmsnorm(nullptr, st->x, w->ln1 + l * H, nullptr, xn, B, H, H, H, w->eps, s);
+      const int sq = gemm_step_partials(xn, H, B, wqkv, NQKV, H, part, room, s);
+      if (sq) {
+        launch_decode_attn_part(part, sq, w->q_norm + l * 128, w->k_norm + l * 128, rope_row,
+                                rope_row + 128, st->pos, kc, vc, B, Hq, Hkv, cap, splits, w->eps,
+                                aw.acc, aw.ml, st->attn, true, s);
+      } else {
+        launch_gemm(xn, H, B, wqkv, NQKV, H, st->qkv, NQKV, nullptr, 0, EPI_NONE, nullptr, nullptr,
+                    nullptr, s);
+        launch_decode_attn(st->qkv, NQKV, w->q_norm + l * 128, w->k_norm + l * 128, rope_row,
+                           rope_row + 128, st->pos, kc, vc, B, Hq, Hkv, cap, splits, w->eps, aw.acc,
+                           aw.ml, st->attn, true, s);
+      }
+      const int so = gemm_step_partials(st->attn, QD, B, wo, H, QD, part, room, s);
+      if (so) {
+        launch_part_add_rmsnorm(part, so, B, st->x, w->ln2 + l * H, xn, H, w->eps, s);
+      } else {
+        launch_gemm(st->attn, QD, B, wo, H, QD, st->x, H, st->x, H, EPI_RES, nullptr, nullptr,
+                    nullptr, s);
+        launch_add_rmsnorm(nullptr, st->x, w->ln2 + l * H, nullptr, xn, B, H, H, H, w->eps, s);
+      }
+      launch_gemm(xn, H, B, wgu, I, H, st->act, I, nullptr, 0, EPI_SWIGLU, nullptr, nullptr, nullptr, s);
+      pend = gemm_step_partials(st->act, I, B, wd, H, I, part, room, s);
+      if (!pend)
+        launch_gemm(st->act, I, B, wd, H, I, st->x, H, st->x, H, EPI_RES, nullptr, nullptr, nullptr, s);
+    }
+    if (pend) {
+      launch_part_add_rmsnorm(part, pend, B, st->x, w->final_norm, lw.xn, H, w->eps, s);
+      return lm_head_normed(lw.xn, lm_weight(w), V, H, B, st->tok, st->pos, lw, s);
+    }
+    return lm_head(st->x, H, lm_weight(w), V, H, B, w->final_norm, w->eps, st->tok, st->pos, nullptr, lw, s);
+  }
   for (int64_t l = 0; l < w->n_layers; ++l) {
     const bf16_t* wqkv = w->w_qkv + l * NQKV * H;
     const bf16_t* wo = w->w_o + l * H * QD;

@@ -83,6 +83,8 @@ bool launch_gemm_skinny(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w,
 // return S; otherwise launch nothing and return 0.
 int gemm_tile_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,
                        int64_t K, float* part, int64_t part_floats, hipStream_t s);
+int gemm_step_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,
+                       int64_t K, float* part, int64_t part_floats, hipStream_t s);
 bool gemm_tile_ok(int64_t M, int64_t N, int64_t K, int epi, const void* x, int64_t x_stride,
                   const void* w, const void* out, int64_t out_stride, const void* res,
                   int64_t res_stride);
@@ -97,12 +99,21 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
                          int64_t K, bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi,
                          float* pval, int32_t* pidx, float* logits, float* part,
                          int64_t part_floats, hipStream_t s);
-// gemm_quad.hip (four-wave MFMA GEMM, 257 and more rows; the LM head from 129 rows)
+// gemm_quad.hip (four-wave MFMA GEMM: 33..64 rows, 257 and more; the LM head there and from 129
+// rows)
 bool launch_gemm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
                       bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi, int splits,
                       int ks_per, float* part, hipStream_t s);
+int quad_small_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
+                        float* part, int64_t part_floats, hipStream_t s);
+int launch_quad_small(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
+                      bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi, float* part,
+                      int64_t part_floats, hipStream_t s);
+int64_t quad_small_ws_floats(int64_t M, int64_t N, int64_t K);
 int64_t launch_lm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
                        float* pval, int32_t* pidx, float* logits, hipStream_t s);
+// rows from which the four-wave kernel's small plan takes over (M <= 32: the skinny kernel)
+constexpr int64_t GEMM_SMALL_MIN_M = 33;
 // rows from which the tiled kernel takes over
 constexpr int64_t GEMM_TILE_MIN_M = 65;
 

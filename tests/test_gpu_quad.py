@@ -79,7 +79,35 @@ def test_split_launches(ops, name, M):
     assert bool(((got - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("name,M", [("qkv", 300), ("gu", 601), ("down", 1500), ("o", 4095)])
+# 33..64 rows: one row block of 64, blocks of 40 to 96 columns, 1 to 8 K splits as the plan and the
+# partial room decide (none: unsplit)
+@pytest.mark.parametrize("name", list(SHAPES))
+@pytest.mark.parametrize("M", [33, 47, 64])
+def test_small_row_counts(ops, name, M):
+    x, w, res = _operands(name, M)
+    N, K = SHAPES[name]
+    acc = x.double() @ w.double().t()
+    a = acc.to(BF).float()
+    for room in (True, False):
+        ws = None if room else torch.zeros(256, dtype=torch.uint8, device="cuda")
+        got = _linear(ops, name, x, w, res, ws=ws).float()
+        if name == "gu":
+            gate, up = a[:, :N], a[:, N:]
+            sg = torch.sigmoid(gate)
+            s = (gate * sg).to(BF).float()
+            want = (s * up).to(BF).float()
+            bound = (up.abs() * ((sg * (1 + gate * (1 - sg))).abs() * bf16_ulp(gate) + bf16_ulp(s))
+                     + s.abs() * bf16_ulp(up) + 2 * bf16_ulp(torch.maximum(got.abs(), want.abs())) + 2 ** -12)
+        elif name == "qkv":
+            want = a
+            bound = 2 * bf16_ulp(torch.maximum(got.abs(), want.abs())) + 2 ** -9
+        else:
+            want = (res.float() + a).to(BF).float()
+            bound = bf16_ulp(a) + 2 * bf16_ulp(torch.maximum(got.abs(), want.abs()))
+        assert bool(((got - want).abs() <= bound).all()), f"room {room}"
+
+
+@pytest.mark.parametrize("name,M", [("gu", 47), ("o", 33), ("qkv", 300), ("gu", 601), ("down", 1500), ("o", 4095)])
 def test_outputs_aligned_to_8_bytes(ops, name, M):
     """An output (and residual) whose rows start 8 bytes off a 16-byte boundary takes the narrow
     stores: the same bits, and nothing written beside the rows."""
@@ -93,3 +121,21 @@ def test_outputs_aligned_to_8_bytes(ops, name, M):
     _linear(ops, name, x, w, r2, out=out)
     assert torch.equal(out, want)
     assert bool((buf[:, :4] == 7).all()) and bool((buf[:, 4 + N:] == 7).all())
+
+
+@pytest.mark.parametrize("B,S,N", [(33, 20, 4), (48, 40, 4), (100, 12, 3), (130, 9, 3)])
+def test_decode_steps_with_split_partials(B, S, N):
+    """Decode steps of more than 32 rows, whose projections leave K-split partials in the LM head's
+    region: greedy ids under the margin rule against the oracle."""
+    from engine import Engine
+    from helpers import ORACLE_TIE, ensure_oracle_built, margin_rule
+    from oracle import qwen3_ref as R
+    from oracle import synth
+    ensure_oracle_built()
+    print(f"\n[case] decode B={B} S={S} N={N}", flush=True)
+    eng = Engine.synthetic(n_layers=2, seed=1)
+    eng.tree_mode = "0"
+    prompt = synth.prompt_ids(60 + B, B, S)
+    toks = torch.tensor(list(eng.generate(prompt.tolist(), N))).numpy().T
+    tl = R.Qwen3Ref.from_synth(1, 2).teacher_logits(prompt, toks)
+    assert margin_rule(toks, tl, margin=ORACLE_TIE, what=f"decode B={B}") == []
