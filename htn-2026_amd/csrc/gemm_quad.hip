@@ -151,6 +151,15 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // The compiler does not see the latency of the asm MFMAs: their results have landed before
+  // anything else may read or copy an accumulator (the main loop copies none).
+  auto settle = [&]() {
+    asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+a"(acc[nt][mt]));
+  };
   // fragments of one K half: NT weight tiles, MT activation tiles, one 16-byte unit per lane each
   struct Frag {
     uint4 v[PER];
@@ -207,24 +216,21 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
     if (toucher) touch(s + NBUF + TOUCH);
     b = bn;
   }
+  settle();
   for (; s + 1 < stages; ++s) {                // the last stages: nothing left to load
     QD_HALF(false, true, f0, f1, b, 1, 0, 0);
     wait_stages<PER, NBUF - 2>(stages - 2 - s);
     lds_barrier();
     const int bn = b + 1 < NBUF ? b + 1 : 0;
     QD_HALF(false, true, f1, f0, bn, 0, 0, 0);
+    settle();
     b = bn;
   }
   QD_HALF(false, true, f0, f1, b, 1, 0, 0);
   QD_HALF(false, false, f1, f0, b, 0, 0, 0);
 #undef QD_HALF
   wait_vm<0>();                                // no load outlives the workgroup
-  // the last MFMAs' results before anything reads them (the compiler does not see their latency)
-  asm volatile("s_nop 15\n\ts_nop 7");
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+a"(acc[nt][mt]));
+  settle();
 
   // epilogue: lane (c, q) of acc[nt][mt] holds four consecutive output columns, of a tile pair
   // eight: columns 32 p + 8 q .. + 7 of the run (an odd last tile: 16 nt + 4 q .. + 3), for
