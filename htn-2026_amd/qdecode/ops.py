@@ -26,7 +26,9 @@ BF16 = torch.bfloat16
 
 
 def stream_ptr():
-    return torch.cuda.current_stream().cuda_stream
+    # the raw handle of torch.cuda.current_stream(), without building its Stream object (2.7 of
+    # the 10 us that a one-row RMSNorm call spent on the host; 0.2 us this way)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
@@ -34,6 +36,9 @@ def _ptr(t):
 
 
 def _check(t, dtype, name, device=None):
+    if (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda
+            and (device is None or t.device == device)):
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.dtype != dtype:
