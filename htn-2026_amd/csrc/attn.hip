@@ -94,6 +94,45 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float* __restrict_
   *reinterpret_cast<uint32_t*>(out + r * 128 + lane * 2) = pack2(y.x, y.y);
 }
 
+// The same merge for at most MS <= 16 splits (merge_splits' single pass, the same bits): four rows
+// per workgroup, every partial row requested before the weights are known.  512 query tokens x 32
+// heads, 2 splits: 7.8 -> 5.6 us; 256 x 32, 8 splits: 7.4 -> 6.7.
+template <int MS>
+__global__ __launch_bounds__(256) void attn_merge_few_kernel(const float* __restrict__ ws_acc,
+                                                             const float* __restrict__ ws_ml,
+                                                             int splits, int64_t rows,
+                                                             bf16_t* __restrict__ out) {
+  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= rows) return;
+  const int lane = threadIdx.x & 63;
+  const float2* acc = reinterpret_cast<const float2*>(ws_acc + r * splits * 128) + lane;
+  float2 a[MS];
+#pragma unroll
+  for (int q = 0; q < MS; ++q) a[q] = acc[(int64_t)(q < splits ? q : splits - 1) * 64];
+  const float2 v = lane < splits ? reinterpret_cast<const float2*>(ws_ml)[r * splits + lane]
+                                 : make_float2(M_FLOOR, 0.f);
+  const float w = __expf(v.x - fmaxf(M_FLOOR, wave_max(v.x)));
+  const float den = wave_sum(w * v.y);
+  float n0 = 0.f, n1 = 0.f;
+#pragma unroll
+  for (int q = 0; q < MS; ++q) {
+    const float wq = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), q));
+    if (q < splits) { n0 = fmaf(wq, a[q].x, n0); n1 = fmaf(wq, a[q].y, n1); }
+  }
+  const float inv = 1.0f / den;
+  *reinterpret_cast<uint32_t*>(out + r * 128 + lane * 2) = pack2(n0 * inv, n1 * inv);
+}
+
+static void launch_attn_merge(const float* ws_acc, const float* ws_ml, int splits, int64_t rows,
+                              bf16_t* out, hipStream_t s) {
+  const dim3 g4((unsigned)((rows + 3) / 4)), b4(256);
+  if (splits <= 2) attn_merge_few_kernel<2><<<g4, b4, 0, s>>>(ws_acc, ws_ml, splits, rows, out);
+  else if (splits <= 4) attn_merge_few_kernel<4><<<g4, b4, 0, s>>>(ws_acc, ws_ml, splits, rows, out);
+  else if (splits <= 8) attn_merge_few_kernel<8><<<g4, b4, 0, s>>>(ws_acc, ws_ml, splits, rows, out);
+  else if (splits <= 16) attn_merge_few_kernel<16><<<g4, b4, 0, s>>>(ws_acc, ws_ml, splits, rows, out);
+  else attn_merge_kernel<<<dim3((unsigned)rows), dim3(64), 0, s>>>(ws_acc, ws_ml, splits, out);
+}
+
 // Split policy: ATTN_NW waves per workgroup take ATTN_TILE keys per iteration.  Splits of at
 // most ATTN_SPLIT_KEYS keys; while (batch x KV heads x splits) < 128 workgroups, more splits
 // (whole tiles) up to ~1 workgroup per CU.  Chosen from a sweep on MI355X of {4, 8} waves x
@@ -144,7 +183,7 @@ void launch_decode_attn(const bf16_t* qkv, int64_t qkv_stride, const bf16_t* qn,
         qkv, qkv_stride, qn, kn, cos_t, sin_t, pos, k_cache, v_cache, Hq, Hkv, cap, chunk, eps,
         1.0f / sqrtf(128.0f), ws_acc, ws_ml, out);
   if (splits > 1)
-    attn_merge_kernel<<<dim3((unsigned)(B * Hq)), dim3(64), 0, s>>>(ws_acc, ws_ml, (int)splits, out);
+    launch_attn_merge(ws_acc, ws_ml, (int)splits, B * Hq, out, s);
 }
 
 // ------------------------------------------------------------------ block (tree / causal chunk)
@@ -569,7 +608,7 @@ void launch_decode_attn_part(const float* part, int part_S, const bf16_t* qn, co
   launch_decode_attn_mfma(nullptr, 0, qn, kn, cos_t, sin_t, pos, k_cache, v_cache, B, Hq, Hkv,
                           cap, splits, chunk, eps, ws_acc, ws_ml, out, rope_row, s, part, part_S);
   if (splits > 1)
-    attn_merge_kernel<<<dim3((unsigned)(B * Hq)), dim3(64), 0, s>>>(ws_acc, ws_ml, (int)splits, out);
+    launch_attn_merge(ws_acc, ws_ml, (int)splits, B * Hq, out, s);
 }
 
 int64_t block_attn_splits(int64_t cap) { return (cap + BLOCK_CHUNK - 1) / BLOCK_CHUNK; }
@@ -638,6 +677,5 @@ void launch_block_attn(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_c
     block_attn_mfma_kernel<true><<<grid, block, 0, s>>>(q, k_cache, v_cache, base, anc, T, Hq, Hkv, cap,
                                                         chunk, scale_log2, ws_acc, ws_ml, out);
   if (use > 1)      // one split writes its rows itself
-    attn_merge_kernel<<<dim3((unsigned)(B * T * Hq)), dim3(64), 0, s>>>(ws_acc, ws_ml, (int)use,
-                                                                        out);
+    launch_attn_merge(ws_acc, ws_ml, (int)use, B * T * Hq, out, s);
 }
