@@ -241,7 +241,20 @@ struct BlockAttnLds {
 };
 
 // CAUSAL: a prompt chunk (anc unused); else ancestor masks.
-template <bool CAUSAL>
+// HALVES: at most 16 RT <= 32 query tokens per sequence (small trees, short chunks).  64-token
+// blocks contract mostly padding there and are bound by that, not by the K/V stream; instead
+// waves w and w + 4 hold the same 16 RT rows and take keys 0..31 and 32..63 of every tile (which
+// also halves the LDS reads: every wave of a 64-token block reads the whole tile), each with its
+// own online softmax, and are combined through LDS at the end.  Measured with q/k norm + RoPE (us):
+//   sequences x tokens, context   64-token blocks -> here
+//   8 x 16, 12000 (tree)          142.0 ->  93.1   (K/V 394 MB: 69 at the 5.7 TB/s of decode attention)
+//   8 x 32, 8000                  105.1 ->  78.7
+//   4 x 16, 8192                   60.2 ->  45.8
+//   2 x 32, 16000                  62.7 ->  51.3
+//   1 x 8, 300                     26.3 ->  18.2
+// and causal chunks alike (8 x 16, 12000: 142.5 -> 93.7).  A fifth tile buffer (160 KB of LDS)
+// gains nothing: 95.7, 80.0, 46.4, 53.1, 18.2.
+template <bool CAUSAL, int RT = 2, bool HALVES = false>
 __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int64_t* __restrict__ base_ptr,
@@ -249,6 +262,7 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
     float scale_log2, float* ws_acc, float* ws_ml, bf16_t* __restrict__ out) {
   typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
   typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+  constexpr int NH = HALVES ? 2 : 4, NJ = NH / 2;           // 16- and 32-key parts of a wave's tile
   __shared__ BlockAttnLds sm;
   const int split = blockIdx.x, kvh = blockIdx.y;
   const int splits = gridDim.x;
@@ -259,15 +273,16 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   const int64_t tb = (QB - 1 - blockIdx.z % QB) * BA_TQ;    // the workgroup's first token
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int head = wave & 3;
-  const int64_t t0 = tb + 32 * (wave >> 2);                 // this wave's first token
+  const int64_t t0 = tb + (HALVES ? 0 : 32 * (wave >> 2));  // this wave's first token
+  const int h0 = HALVES ? 2 * (wave >> 2) : 0;              // and first 16-key part
   const int c = lane & 15, q4 = lane >> 4;
   const int64_t base = base_ptr[b];
   // query rows of this lane: token t0 + 16 rt + c, head kvh * 4 + head
-  uint4 qf[2][4];
-  uint64_t mask[2];
-  int64_t tok[2];
+  uint4 qf[RT][4];
+  uint64_t mask[RT];
+  int64_t tok[RT];
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     tok[rt] = t0 + 16 * rt + c;
     const int64_t tt = tok[rt] < T ? tok[rt] : T - 1;
     const uint4* qr = reinterpret_cast<const uint4*>(q + ((b * T + tt) * Hq + kvh * GRP + head) * 128);
@@ -286,12 +301,15 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   const uint4* vb = reinterpret_cast<const uint4*>(v_cache + head_off);
   // o[rt][dt]: O^T dims 16 dt + 4 q4 .. + 3 of the lane's row c; lsum[rt]: the fp32 sum of the
   // lane's probabilities of that row (its four q lanes hold disjoint keys)
-  float m[2] = {M_FLOOR, M_FLOOR}, lsum[2] = {0.f, 0.f};
-  f32x4_t o[2][8];
+  float m[RT], lsum[RT];
+  f32x4_t o[RT][8];
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+  for (int rt = 0; rt < RT; ++rt) {
+    m[rt] = M_FLOOR;
+    lsum[rt] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) o[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
   // Staging by DMA (global_load_lds_dwordx4, no registers): wave w moves the 1 KiB blocks 2w
   // and 2w + 1 of a tile's K and of its V (block j = keys 4j .. 4j + 3); lane l of block j lands
   // in LDS slot 64 j + l = unit (l & 15) of key 4 j + (l >> 4) as stored, i.e. logical unit
@@ -322,19 +340,19 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
     }
   };
   // S' of the tile in `buf` for both row tiles: sc[rt][h] = keys 16 h + 4 q4 .. + 3, row c
-  auto scores = [&](int buf, f32x4_t (&sc)[2][4]) {
+  auto scores = [&](int buf, f32x4_t (&sc)[RT][NH]) {
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int h = 0; h < 4; ++h) sc[rt][h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int h = 0; h < NH; ++h) sc[rt][h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      const int key = 16 * h + c;                            // key & 15 == c
+    for (int h = 0; h < NH; ++h) {
+      const int key = 16 * (h0 + h) + c;                            // key & 15 == c
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
         const uint4 kf = sm.k[buf][key * 16 + ((4 * kk + q4) ^ c)];
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
           sc[rt][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               __builtin_bit_cast(bf16x8_t, kf), __builtin_bit_cast(bf16x8_t, qf[rt][kk]),
               sc[rt][h], 0, 0, 0);
@@ -345,13 +363,13 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   // visibility word per row (bit i = tile key j0 + i): the tile's cached keys (below base), the
   // block keys the row sees (its ancestor bits, or for a causal chunk the keys up to itself),
   // cut at kend
-  auto mask_tile = [&](int64_t j0, f32x4_t (&sc)[2][4]) {
+  auto mask_tile = [&](int64_t j0, f32x4_t (&sc)[RT][NH]) {
     const int jrel0 = (int)(j0 - base);                       // block index of key j0 (may be < 0)
     const int lim = (int)(kend - j0);                         // keys of the tile below kend
     const uint64_t limbits = lim >= 64 ? ~0ull : lim <= 0 ? 0ull : (1ull << lim) - 1;
     const uint64_t cached = jrel0 >= 0 ? 0ull : jrel0 <= -64 ? ~0ull : (1ull << -jrel0) - 1;
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
       uint64_t blk;
       if constexpr (!CAUSAL) {
         blk = jrel0 >= 64 ? 0ull : jrel0 >= 0 ? mask[rt] >> jrel0
@@ -362,8 +380,8 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
       }
       const uint64_t vis = (cached | blk) & limbits;
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const uint32_t nib = (uint32_t)(vis >> (16 * h + 4 * q4)) & 15u;
+      for (int h = 0; h < NH; ++h) {
+        const uint32_t nib = (uint32_t)(vis >> (16 * (h0 + h) + 4 * q4)) & 15u;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (!((nib >> r) & 1u)) sc[rt][h][r] = NEG_INF;
@@ -372,24 +390,26 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   };
   // softmax of a tile's scores: rescale O / l if a row's maximum jumped, then the tile's
   // probabilities as bf16 MFMA B fragments pf (keys 8 j .. 8 j + 7 of the lane's order)
-  auto softmax = [&](const f32x4_t (&sc)[2][4], uint4 (&pf)[2][2]) {
-    float mx[2];
-    bool need[2];
+  auto softmax = [&](const f32x4_t (&sc)[RT][NH], uint4 (&pf)[RT][NJ]) {
+    float mx[RT];
+    bool need[RT], any = false;
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      float x[4];
+    for (int rt = 0; rt < RT; ++rt) {
+      float x[NH];
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
+      for (int h = 0; h < NH; ++h)
         x[h] = fmaxf(fmaxf(sc[rt][h][0], sc[rt][h][1]), fmaxf(sc[rt][h][2], sc[rt][h][3]));
-      float y = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+      float y = fmaxf(x[0], x[1]);
+      if constexpr (NH == 4) y = fmaxf(y, fmaxf(x[2], x[3]));
       y = fmaxf(y, lane_xor16(y));
       y = fmaxf(y, lane_xor32(y));
       mx[rt] = y * scale_log2;                                // = max of the scaled scores
       need[rt] = mx[rt] > m[rt] + BA_TAU;
+      any = any || need[rt];
     }
-    if (__ballot(need[0] || need[1]) != 0) {                 // wave-uniform
+    if (__ballot(any) != 0) {                 // wave-uniform
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
+      for (int rt = 0; rt < RT; ++rt) {
         const float mn = need[rt] ? mx[rt] : m[rt];
         const float a = __builtin_amdgcn_exp2f(m[rt] - mn);  // 1 for rows that keep m
         m[rt] = mn;
@@ -399,21 +419,24 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
       }
     }
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      float p[16];
+    for (int rt = 0; rt < RT; ++rt) {
+      float p[4 * NH];
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
+      for (int h = 0; h < NH; ++h)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           p[4 * h + r] = __builtin_amdgcn_exp2f(fmaf(sc[rt][h][r], scale_log2, -m[rt]));
       float t[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) t[e] = p[e] + p[e + 8];
+      for (int e = 0; e < 8; ++e) {
+        t[e] = p[e];
+        if constexpr (NH == 4) t[e] += p[e + 8];
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) t[e] += t[e + 4];
       lsum[rt] += (t[0] + t[2]) + (t[1] + t[3]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NJ; ++j)
         pf[rt][j] = make_uint4(pack2(p[8 * j + 0], p[8 * j + 1]), pack2(p[8 * j + 2], p[8 * j + 3]),
                                pack2(p[8 * j + 4], p[8 * j + 5]), pack2(p[8 * j + 6], p[8 * j + 7]));
     }
@@ -427,16 +450,16 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   };
   // O^T += V^T . P^T from the tile in `buf`, per 32-key half j: keys 32 j + 4 q4 .. + 3 and
   // 32 j + 16 + 4 q4 .. + 3
-  auto pv = [&](int buf, const uint4 (&pf)[2][2]) {
+  auto pv = [&](int buf, const uint4 (&pf)[RT][NJ]) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) {
-        const uint2 lo = lds_read_tr16(vt_addr(buf, dt, 2 * j));
-        const uint2 hi = lds_read_tr16(vt_addr(buf, dt, 2 * j + 1));
+        const uint2 lo = lds_read_tr16(vt_addr(buf, dt, h0 + 2 * j));
+        const uint2 hi = lds_read_tr16(vt_addr(buf, dt, h0 + 2 * j + 1));
         const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
           o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               __builtin_bit_cast(bf16x8_t, vf), __builtin_bit_cast(bf16x8_t, pf[rt][j]),
               o[rt][dt], 0, 0, 0);
@@ -458,8 +481,8 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   wait_vm<4 * (AHEAD - 1)>();
   lds_barrier();
   const bool lead = wave < 4;                                // wave-uniform
-  f32x4_t sc[2][4];
-  uint4 pf[2][2];
+  f32x4_t sc[RT][NH];
+  uint4 pf[RT][NJ];
   // a tile is visible to every row of the workgroup when it ends below kend and below base --
   // or, in a causal chunk, below the workgroup's first token (every row sees the block keys
   // before it)
@@ -520,8 +543,35 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
     pv(bprev, pf);
   }
   wait_vm<0>();                                              // no DMA outlives the workgroup
+  if constexpr (HALVES) {
+    // waves 4-7 hand their (m, l, O) over, waves 0-3 (the same rows) fold them in
+    f32x4_t* ho = reinterpret_cast<f32x4_t*>(&sm.k[0][0]) + head * RT * 8 * 64 + lane;
+    float2* hml = reinterpret_cast<float2*>(reinterpret_cast<f32x4_t*>(&sm.k[0][0]) + 4 * RT * 8 * 64) +
+                  head * RT * 64 + lane;
+    lds_barrier();                                           // every wave is done with the tiles
+    if (!lead) {
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
+      for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) ho[(rt * 8 + dt) * 64] = o[rt][dt];
+        hml[rt * 64] = make_float2(m[rt], lsum[rt]);
+      }
+    }
+    lds_barrier();
+    if (!lead) return;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const float2 z = hml[rt * 64];
+      const float mn = fmaxf(m[rt], z.x);
+      const float a = __builtin_amdgcn_exp2f(m[rt] - mn), az = __builtin_amdgcn_exp2f(z.x - mn);
+      m[rt] = mn;
+      lsum[rt] = lsum[rt] * a + z.y * az;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) o[rt][dt] = o[rt][dt] * a + ho[(rt * 8 + dt) * 64] * az;
+    }
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
     float l = lsum[rt];
     l += lane_xor16(l);
     l += lane_xor32(l);
@@ -670,12 +720,22 @@ void launch_block_attn(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_c
   const int64_t chunk = ((cap + use - 1) / use + 31) / 32 * 32;
   const dim3 grid((unsigned)use, (unsigned)Hkv, (unsigned)(B * QB)), block(512);
   const float scale_log2 = (1.0f / sqrtf(128.0f)) * 1.44269504088896341f;
-  if (anc)
-    block_attn_mfma_kernel<false><<<grid, block, 0, s>>>(q, k_cache, v_cache, base, anc, T, Hq, Hkv, cap,
-                                                         chunk, scale_log2, ws_acc, ws_ml, out);
-  else
-    block_attn_mfma_kernel<true><<<grid, block, 0, s>>>(q, k_cache, v_cache, base, anc, T, Hq, Hkv, cap,
-                                                        chunk, scale_log2, ws_acc, ws_ml, out);
+#define QD_BLOCK(...)                                                                           \
+  block_attn_mfma_kernel<__VA_ARGS__><<<grid, block, 0, s>>>(q, k_cache, v_cache, base, anc, T, Hq, Hkv, \
+                                                             cap, chunk, scale_log2, ws_acc, ws_ml, out)
+  // up to 32 tokens the half-tile form (its comment has both sides measured); from 33 a block's
+  // second 16-row pair is in use and every row tile of the 64-token form counts
+  if (T <= 16) {
+    if (anc) QD_BLOCK(false, 1, true);
+    else QD_BLOCK(true, 1, true);
+  } else if (T <= 32) {
+    if (anc) QD_BLOCK(false, 2, true);
+    else QD_BLOCK(true, 2, true);
+  } else {
+    if (anc) QD_BLOCK(false);
+    else QD_BLOCK(true);
+  }
+#undef QD_BLOCK
   if (use > 1)      // one split writes its rows itself
     launch_attn_merge(ws_acc, ws_ml, (int)use, B * T * Hq, out, s);
 }
