@@ -233,6 +233,7 @@ constexpr int BA_NBUF = QD_BA_NBUF;   // LDS tile buffers (BA_NBUF - 3 tiles in 
 #define QD_BA_TAU 8.0f
 #endif
 constexpr float BA_TAU = QD_BA_TAU;
+constexpr int64_t BA_HALVES_CHUNK = 640;
 constexpr float BA_LN2 = 0.69314718055994531f;
 
 struct BlockAttnLds {
@@ -241,7 +242,7 @@ struct BlockAttnLds {
 };
 
 // CAUSAL: a prompt chunk (anc unused); else ancestor masks.
-// HALVES: at most 16 RT <= 32 query tokens per sequence (small trees, short chunks).  64-token
+// HALVES: at most 16 RT <= 48 query tokens per sequence (small trees, short chunks).  64-token
 // blocks contract mostly padding there and are bound by that, not by the K/V stream; instead
 // waves w and w + 4 hold the same 16 RT rows and take keys 0..31 and 32..63 of every tile (which
 // also halves the LDS reads: every wave of a 64-token block reads the whole tile), each with its
@@ -254,6 +255,10 @@ struct BlockAttnLds {
 //   1 x 8, 300                     26.3 ->  18.2
 // and causal chunks alike (8 x 16, 12000: 142.5 -> 93.7).  A fifth tile buffer (160 KB of LDS)
 // gains nothing: 95.7, 80.0, 46.4, 53.1, 18.2.
+// 33 to 48 tokens (RT = 3, 256 registers; four row tiles would spill) save a quarter of the
+// contraction and pay ~1 us for the combination: 8 x 48, 8000 (splits of 2048 keys) 108.7 ->
+// 96.7, 4 x 40, 8192 (1056) 65.7 -> 62.2, but 1 x 48, 2000 (416) 30.7 -> 31.2 and 8 x 33, 1000
+// (384) 33.5 -> 34.0, so only splits of BA_HALVES_CHUNK keys and more take it.
 template <bool CAUSAL, int RT = 2, bool HALVES = false>
 __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
@@ -723,14 +728,17 @@ void launch_block_attn(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_c
 #define QD_BLOCK(...)                                                                           \
   block_attn_mfma_kernel<__VA_ARGS__><<<grid, block, 0, s>>>(q, k_cache, v_cache, base, anc, T, Hq, Hkv, \
                                                              cap, chunk, scale_log2, ws_acc, ws_ml, out)
-  // up to 32 tokens the half-tile form (its comment has both sides measured); from 33 a block's
-  // second 16-row pair is in use and every row tile of the 64-token form counts
+  // up to 32 tokens the half-tile form (its comment has both sides measured), up to 48 where a
+  // split is long enough to pay for combining three row tiles
   if (T <= 16) {
     if (anc) QD_BLOCK(false, 1, true);
     else QD_BLOCK(true, 1, true);
   } else if (T <= 32) {
     if (anc) QD_BLOCK(false, 2, true);
     else QD_BLOCK(true, 2, true);
+  } else if (T <= 48 && chunk >= BA_HALVES_CHUNK) {
+    if (anc) QD_BLOCK(false, 3, true);
+    else QD_BLOCK(true, 3, true);
   } else {
     if (anc) QD_BLOCK(false);
     else QD_BLOCK(true);

@@ -1,5 +1,6 @@
-"""Block attention of at most 32 query tokens (attn.hip, HALVES): the edges of its row tiles and of
-the 64-key tiles whose halves different waves take, with one key split and several."""
+"""Block attention of at most 48 query tokens (attn.hip, HALVES): the edges of its row tiles and of
+the 64-key tiles whose halves different waves take, with one key split and several, short
+splits and long ones."""
 
 import math
 
@@ -25,8 +26,8 @@ def _masks(B, T, tree, g):
 
 
 @pytest.mark.parametrize("tree", [True, False])
-@pytest.mark.parametrize("T", [1, 15, 16, 17, 31, 32, 33])
-@pytest.mark.parametrize("B,base,spare", [(1, 0, 0), (2, 31, 5), (3, 33, 700), (2, 1500, 0), (9, 64, 3)])
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 31, 32, 33, 47, 48, 49])
+@pytest.mark.parametrize("B,base,spare", [(1, 0, 0), (2, 31, 5), (3, 33, 700), (2, 1500, 0), (9, 64, 3), (9, 2100, 3)])
 def test_small_blocks(B, base, spare, T, tree):
     from qdecode import ops
     print(f"\n[case] B={B} T={T} base={base} spare={spare} tree={tree}", flush=True)
