@@ -713,6 +713,23 @@ int64_t gemm_tile_ws_floats(int64_t M, int64_t N, int64_t K, int epi) {
   return sp > 1 ? (int64_t)sp * M * N : 0;
 }
 
+// Falls with the row count as well as growing with it: from 33 to 64 rows the plan takes fewer splits
+// as rows are added, and past that the split count drops where a 128-row block is added (one count
+// per number of blocks, so a block's largest need is at its last row count).
+int64_t gemm_tile_ws_floats_upto(int64_t B, int64_t T, int64_t N, int64_t K, int epi) {
+  int64_t most = 0;
+  auto take = [&](int64_t t) {
+    const int64_t f = gemm_tile_ws_floats(B * t, N, K, epi);
+    if (f > most) most = f;
+  };
+  for (int64_t t = (GEMM_SMALL_MIN_M + B - 1) / B; t <= T && B * t < GEMM_TILE_MIN_M; ++t) take(t);
+  for (int64_t rows = TM;; rows += TM) {
+    const int64_t t = rows / B < T ? rows / B : T;
+    if (B * t >= GEMM_TILE_MIN_M) take(t);
+    if (t == T || gemm_tile_splits(rows, N, K, epi) <= 1) return most;
+  }
+}
+
 // as gemm_tile_partials, for a decode step's rows: where the all-rows kernel's split count does
 // not fit part_floats, the four-wave kernel takes fewer
 int gemm_step_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,

@@ -629,31 +629,42 @@ int qd_mega_step(const qd_weights* w, const qd_decode_state* st, void* stream) {
 }
 
 // ------------------------------------------------------------------ block (tree / prefill chunk)
-// split-K partials of the block step's projections (the largest of qkv, o, down)
-static int64_t block_part_floats(const qd_weights* w, int64_t M) {
+// split-K partials of the block step's projections (the largest of qkv, o, down) at B T rows, or
+// with `upto` the largest over every T' <= T
+static int64_t block_part_floats(const qd_weights* w, int64_t B, int64_t T, bool upto) {
   const int64_t H = w->hidden, QD = (int64_t)w->n_q_heads * 128;
-  int64_t f = gemm_tile_ws_floats(M, qkv_width(w), H, EPI_NONE);
-  const int64_t o = gemm_tile_ws_floats(M, H, QD, EPI_RES);
-  const int64_t d = gemm_tile_ws_floats(M, H, w->inter, EPI_RES);
+  auto need = [&](int64_t N, int64_t K, int epi) {
+    return upto ? gemm_tile_ws_floats_upto(B, T, N, K, epi) : gemm_tile_ws_floats(B * T, N, K, epi);
+  };
+  int64_t f = need(qkv_width(w), H, EPI_NONE);
+  const int64_t o = need(H, QD, EPI_RES);
+  const int64_t d = need(H, w->inter, EPI_RES);
   if (o > f) f = o;
   if (d > f) f = d;
   return f;
 }
 
+static int64_t block_bytes(const qd_weights* w, int64_t B, int64_t T, int64_t cap, int32_t lm_mode,
+                           int64_t part_floats) {
+  // LM-head region first: partials for every row (QD_LM_ALL) or the last row per sequence
+  Carver c(nullptr);
+  carve_lm(c, lm_mode == QD_LM_ALL ? B * T : B, w->vocab, w->hidden);
+  // attention split partials only for the row counts whose launches split the keys (a tree
+  // verification; a prefill chunk of >= 1024 rows runs one split and needs none)
+  const int64_t rows = block_attn_partial_rows(B, T, w->n_q_heads, w->n_kv_heads, cap);
+  c.take<float>(rows * 128);
+  c.take<float>(rows * 2);
+  c.take<float>(part_floats);
+  return c.off;
+}
+
+// Enough for every T' <= T: a runner keeps one workspace for its largest T.  (A step asks for what
+// its own T needs, no more.)
 int64_t qd_block_workspace_bytes_lm(const qd_weights* w, int64_t batch, int64_t T, int64_t cap,
                                     int32_t lm_mode) {
   if (!w || batch <= 0 || T <= 0 || cap <= 0 || lm_mode < QD_LM_ALL || lm_mode > QD_LM_NONE)
     return 0;
-  // LM-head region first: partials for every row (QD_LM_ALL) or the last row per sequence
-  Carver c(nullptr);
-  carve_lm(c, lm_mode == QD_LM_ALL ? batch * T : batch, w->vocab, w->hidden);
-  // attention split partials only for the row counts whose launches split the keys (a tree
-  // verification; a prefill chunk of >= 1024 rows runs one split and needs none)
-  const int64_t rows = block_attn_partial_rows(batch, T, w->n_q_heads, w->n_kv_heads, cap);
-  c.take<float>(rows * 128);
-  c.take<float>(rows * 2);
-  c.take<float>(block_part_floats(w, batch * T));
-  return c.off;
+  return block_bytes(w, batch, T, cap, lm_mode, block_part_floats(w, batch, T, true));
 }
 
 int64_t qd_block_workspace_bytes(const qd_weights* w, int64_t batch, int64_t T, int64_t cap) {
@@ -671,7 +682,8 @@ int qd_block_step(const qd_weights* w, const qd_block_state* st, void* stream) {
     return QD_EARG;
   if (!st->causal && (!st->anc || !st->depth || T > 64)) return QD_EARG;
   if (block_attn_splits(cap) > 1024) return QD_EARG;
-  if (!st->workspace || st->workspace_bytes < qd_block_workspace_bytes_lm(w, B, T, cap, st->lm_mode))
+  const int64_t part_floats = block_part_floats(w, B, T, false);
+  if (!st->workspace || st->workspace_bytes < block_bytes(w, B, T, cap, st->lm_mode, part_floats))
     return QD_EWS;
   hipStream_t s = S(stream);
   const int64_t M = B * T;
@@ -681,7 +693,6 @@ int qd_block_step(const qd_weights* w, const qd_block_state* st, void* stream) {
   const int64_t arows = block_attn_partial_rows(B, T, Hq, Hkv, cap);
   float* acc = c.take<float>(arows * 128);
   float* ml = c.take<float>(arows * 2);
-  const int64_t part_floats = block_part_floats(w, M);
   float* part = c.take<float>(part_floats);
   const int64_t NQKV = qkv_width(w), QD = (int64_t)Hq * 128;
   const int64_t layer_kv = B * Hkv * cap * 128;

@@ -95,6 +95,8 @@ int gemm_tile_splits(int64_t M, int64_t N, int64_t K, int epi);
 int gemm_rows_query(int64_t M, int64_t N, int64_t K, int epi, bool partials_only,
                     int64_t part_floats, int64_t* out);
 int64_t gemm_tile_ws_floats(int64_t M, int64_t N, int64_t K, int epi);
+// the most it asks for over B t rows, 1 <= t <= T
+int64_t gemm_tile_ws_floats_upto(int64_t B, int64_t T, int64_t N, int64_t K, int epi);
 int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,
                          int64_t K, bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi,
                          float* pval, int32_t* pidx, float* logits, float* part,

@@ -123,6 +123,23 @@ def test_block_workspace_sizes(lib):
     assert L.qd_block_workspace_bytes_lm(C.byref(w), 4, 64, 8512, 3) == 0              # bad mode
 
 
+def test_block_workspace_covers_smaller_blocks(lib):
+    """A runner keeps one workspace, sized for its largest T: no smaller T may ask for more, also
+    where the projections' K split count falls as rows are added (33..64 rows, whole 128-row
+    blocks)."""
+    L = lib.LIB
+    w = lib.Weights(36, 2560, 9728, 151936, 32, 8, 128, 1e-6, *([256] * 10))
+    for cap in (119, 768, 40000):
+        for B, t_end in ((1, 1100), (2, 600), (3, 400), (4, 300), (7, 120), (40, 8)):
+            for mode in (lib.LM_ALL, lib.LM_LAST, lib.LM_NONE):
+                most = 0
+                for T in range(1, t_end):
+                    n = L.qd_block_workspace_bytes_lm(C.byref(w), B, T, cap, mode)
+                    assert n >= most, (B, T, cap, mode)
+                    most = n
+                assert L.qd_block_workspace_bytes_lm(C.byref(w), B, 32768, cap, mode) >= most
+
+
 def test_missing_library_raises(tmp_path):
     """The product path has no fallback: a missing library is an ImportError."""
     import subprocess

@@ -168,6 +168,21 @@ def test_prefill_chunking_is_invariant(eng4, ref4):
             assert np.array_equal(toks[b, :first_tie], outs[2][b, :first_tie]), (b, outs)
 
 
+def test_prefill_tail_below_the_runner_size(eng4, ref4):
+    """A prompt whose last chunk has fewer rows than the prefill runner is sized for, at row counts
+    where the smaller chunk asks for more split partials: 60 + 55 rows, and 800 + 700."""
+    for S, rows, N in ((115, 60, 4), (1500, 800, 3)):
+        say(f"prompt of {S} in chunks of {rows} rows")
+        p = synth.prompt_ids(15, 1, S)
+        eng4.prefill_budget_rows = rows
+        eng4.shape = None
+        toks = np.array(list(eng4.generate(p.tolist(), N))).T
+        eng4.prefill_budget_rows = None
+        eng4.shape = None
+        assert margin_rule(toks, ref4.teacher_logits(p, toks), margin=ORACLE_TIE,
+                           what=f"{S} in {rows}") == []
+
+
 @pytest.fixture(scope="module")
 def eng2(Engine):
     say("Engine.synthetic(2 layers, seed 1)")
