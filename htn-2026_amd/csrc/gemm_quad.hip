@@ -48,8 +48,17 @@ constexpr int TK = 64;                         // K per stage: 128 bytes of ever
 #define QD_QUAD_GROUP_M 4   // M blocks per group of the tile order
 #endif
 
+// WAIT: the 8 wait states that a VALU read of the result needs, in the same asm.  The compiler does
+// not see the latency of an MFMA in asm and may copy an accumulator right behind one (it does where
+// the main loop's accumulators become the tail's), so the last MFMA of a K half carries them; the
+// others are followed by an MFMA and the rest of that wait.
+template <bool WAIT>
 __device__ __forceinline__ void mfma_acc(f32x4_t& acc, uint4 a, uint4 b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(as_bf8(a)), "v"(as_bf8(b)));
+  if constexpr (WAIT)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 7"
+                 : "+a"(acc) : "v"(as_bf8(a)), "v"(as_bf8(b)));
+  else
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(as_bf8(a)), "v"(as_bf8(b)));
 }
 
 // one dword per lane into LDS (256 bytes at lds): brings the lanes' lines into this XCD's L2
@@ -151,10 +160,11 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // The compiler does not see the latency of the asm MFMAs: their results have landed before
-  // anything else may read or copy an accumulator (the main loop copies none).
+  // After a loop and at the end: the accumulators stay where they are until the last MFMA (with its
+  // wait) is behind, and what the compiler has moved at a loop's end is two wait states old before
+  // an MFMA reads it.
   auto settle = [&]() {
-    asm volatile("s_nop 15\n\ts_nop 7");
+    asm volatile("s_nop 1");
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -185,8 +195,10 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
     if (LD) load(st, lb, g_);                                                                  \
     if (RD) rd(nxt, rb, hf, g_);                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                         \
-    _Pragma("unroll") for (int e_ = g_ * MT * NT / PER; e_ < (g_ + 1) * MT * NT / PER; ++e_)   \
-      mfma_acc(acc[e_ % NT][e_ / NT], cur.v[e_ % NT], cur.v[NT + e_ / NT]);                    \
+    _Pragma("unroll") for (int e_ = g_ * MT * NT / PER; e_ < (g_ + 1) * MT * NT / PER; ++e_) { \
+      if (e_ + 1 < MT * NT) mfma_acc<false>(acc[e_ % NT][e_ / NT], cur.v[e_ % NT], cur.v[NT + e_ / NT]); \
+      else mfma_acc<true>(acc[e_ % NT][e_ / NT], cur.v[e_ % NT], cur.v[NT + e_ / NT]);         \
+    }                                                                                          \
     __builtin_amdgcn_sched_barrier(0);                                                         \
   }
 #pragma unroll
