@@ -550,9 +550,11 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   wait_vm<0>();                                              // no DMA outlives the workgroup
   if constexpr (HALVES) {
     // waves 4-7 hand their (m, l, O) over, waves 0-3 (the same rows) fold them in
-    f32x4_t* ho = reinterpret_cast<f32x4_t*>(&sm.k[0][0]) + head * RT * 8 * 64 + lane;
-    float2* hml = reinterpret_cast<float2*>(reinterpret_cast<f32x4_t*>(&sm.k[0][0]) + 4 * RT * 8 * 64) +
-                  head * RT * 64 + lane;
+    static_assert(4 * RT * 64 * (8 * sizeof(f32x4_t) + sizeof(float2)) <= sizeof(BlockAttnLds),
+                  "the hand-over lies over the tile buffers, K's and V's");
+    f32x4_t* const hand = reinterpret_cast<f32x4_t*>(&sm);
+    f32x4_t* ho = hand + head * RT * 8 * 64 + lane;
+    float2* hml = reinterpret_cast<float2*>(hand + 4 * RT * 8 * 64) + head * RT * 64 + lane;
     lds_barrier();                                           // every wave is done with the tiles
     if (!lead) {
 #pragma unroll
