@@ -271,6 +271,7 @@ bool skinny_ok(int64_t M, int64_t N, int64_t K, int epi, int S, const void* x, i
   if (K % SK_KC || N % 4 || N >= (1 << 30) || K >= (1 << 30)) return false;
   if (K / SK_KC < S) return false;
   if (xs % 8 || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16) return false;
+  if (M * xs * 2 >= (1ll << 32)) return false;       // the activations' buffer extent is 32-bit bytes
   if (os % 4) return false;
   const int64_t rows = skinny_rows(N, S);
   return (rows + 15) / 16 <= (epi == EPI_SWIGLU ? 3 : 4);

@@ -645,6 +645,9 @@ static int rows_launch_plan(int64_t M, int64_t N, int64_t K, int epi, bool parti
   return P.splits > 0 ? 1 : -1;
 }
 
+// the all-rows kernel's activation row offsets are 32-bit bytes
+static bool rows_stride_ok(int64_t M, int64_t xs, int64_t K) { return ((M - 1) * xs + K) * 2 < (1ll << 32); }
+
 template <int EPI, bool SPLIT>
 static void launch_rows(const RowsPlan& P, const bf16_t* x, int64_t xs, int M, const bf16_t* w,
                         int N, int K, bf16_t* out, int64_t os, const bf16_t* res, int64_t rs,
@@ -747,7 +750,7 @@ int gemm_tile_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
     return 0;
   if (M < GEMM_TILE_MIN_M) return quad_small_partials(x, xs, M, w, N, K, part, part_floats, s);
   RowsPlan P;
-  const int rp = rows_launch_plan(M, N, K, EPI_NONE, true, part_floats, P);
+  const int rp = rows_stride_ok(M, xs, K) ? rows_launch_plan(M, N, K, EPI_NONE, true, part_floats, P) : -1;
   if (rp == 0) return 0;
   if (rp == 1) {
     launch_rows<EPI_NONE, true>(P, x, xs, (int)M, w, (int)N, (int)K, nullptr, 0, nullptr, 0,
@@ -790,7 +793,8 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
     if (S >= 0) return 0;
   }
   RowsPlan P;
-  if (epi != EPI_ARGMAX && rows_launch_plan(M, N, K, epi, false, part ? part_floats : 0, P) == 1) {
+  if (epi != EPI_ARGMAX && rows_stride_ok(M, xs, K) &&
+      rows_launch_plan(M, N, K, epi, false, part ? part_floats : 0, P) == 1) {
     if (P.splits > 1) {
       launch_rows<EPI_NONE, true>(P, x, xs, (int)M, w, (int)N, (int)K, nullptr, 0, nullptr, 0,
                                   part, s);
