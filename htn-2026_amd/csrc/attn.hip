@@ -677,24 +677,11 @@ int64_t block_attn_splits(int64_t cap) { return (cap + BLOCK_CHUNK - 1) / BLOCK_
 // covering a whole number of 32-key tiles.  Measured on MI355X (config 5): 17 splits of 512
 // keys (544 workgroups, a 1/8-full third round) 10.44 ms per verify forward, 16 splits 9.66 ms,
 // 8 splits 9.08 ms; the 4 x 8192 prefill 0.69 -> 0.59 s with one split instead of 17.
-static int64_t block_attn_cus() {
-  static int64_t cus = -1;
-  if (cus < 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cus = n > 0 ? n : 256;
-  }
-  return cus;
-}
 
 int64_t block_attn_launch_splits(int64_t B, int64_t T, int Hkv, int64_t cap) {
   const int64_t QB = (T + BA_TQ - 1) / BA_TQ;
   const int64_t blocks = (int64_t)Hkv * B * QB;
-  int64_t use = block_attn_cus() / (blocks > 0 ? blocks : 1);
+  int64_t use = plan_cus() / (blocks > 0 ? blocks : 1);
   const int64_t most = block_attn_splits(cap);
   if (use > most) use = most;
   if (use < 1) use = 1;

@@ -385,19 +385,6 @@ __global__ __launch_bounds__(256) void add_rmsnorm_rows_kernel(
   }
 }
 
-static int64_t arn_cus() {
-  static int64_t cus = -1;
-  if (cus < 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cus = n > 0 ? n : 256;
-  }
-  return cus;
-}
 
 // add_rmsnorm_kernel for 256 < hidden / 8 <= 512 with both chunks' loads issued first (as
 // part_add_rmsnorm2_kernel; same arithmetic, same bits).
@@ -451,7 +438,7 @@ void launch_add_rmsnorm(const bf16_t* x, const bf16_t* res, const bf16_t* w, bf1
                         bf16_t* y, int64_t rows, int64_t hidden, int64_t in_stride,
                         int64_t y_stride, float eps, hipStream_t s) {
   if (rows <= 0) return;
-  const int64_t grid = arn_cus() * QD_ARN_WG_PER_CU;
+  const int64_t grid = plan_cus() * QD_ARN_WG_PER_CU;
   if (rows > grid && hidden / 8 <= 256 * ARN_J) {
     if (x)
       add_rmsnorm_rows_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, s>>>(

@@ -536,19 +536,7 @@ static void gemm_lds_go(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w,
 }
 
 // one workgroup per CU
-static int stream_grid() {
-  static int grid = -1;
-  if (grid < 0) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-      (void)hipGetLastError();
-      cus = 0;
-    }
-    grid = cus;
-  }
-  return grid;
-}
+static int stream_grid() { return device_cus(); }
 
 template <int MT, int EPI, int G>
 static void stream_go(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,

@@ -390,19 +390,6 @@ constexpr bool quad_fits() {
 }
 static_assert(quad_fits(), "the CU's LDS");
 
-int64_t quad_cus() {
-  static int64_t cus = -1;
-  if (cus < 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cus = n > 0 ? n : 256;
-  }
-  return cus;
-}
 
 int quad_plan(int64_t M, int64_t N, bool sw, int64_t splits, int64_t stages) {
   int best = -1;
@@ -412,7 +399,7 @@ int quad_plan(int64_t M, int64_t N, bool sw, int64_t splits, int64_t stages) {
     if (sw && q.nt % 2) continue;
     const int64_t bm = 32 * q.mt, bn = quad_outs(q.nt, sw);
     const int64_t wgs = (M + bm - 1) / bm * ((N + bn - 1) / bn) * splits;
-    const double t = (double)((wgs + quad_cus() - 1) / quad_cus()) *
+    const double t = (double)((wgs + plan_cus() - 1) / plan_cus()) *
                      (q.a + (sw ? QUAD_SWIGLU * q.mt * q.nt : 0.0) + (double)q.b * stages);
     if (best < 0 || t < best_t) {
       best = i;
@@ -504,12 +491,12 @@ static SmallPlan quad_small_plan(int64_t M, int64_t N, int64_t K, bool sw, int64
     for (int nt = 2; nt <= 6; ++nt) {
       if (nt == 5 || (sw && nt % 2)) continue;
       const int64_t most = quad_outs(nt, sw);
-      const int64_t blocks = quad_cus() / (S * mbl) > 0 ? quad_cus() / (S * mbl) : 1;   // one round
+      const int64_t blocks = plan_cus() / (S * mbl) > 0 ? plan_cus() / (S * mbl) : 1;   // one round
       int64_t outs = ((N + blocks - 1) / blocks + 7) / 8 * 8;
       if (outs > most) outs = most;
       const int64_t wgs = (N + outs - 1) / outs * S * mbl;
       const double rows = (double)outs * (sw ? 2 : 1);
-      const double t = (double)((wgs + quad_cus() - 1) / quad_cus()) *
+      const double t = (double)((wgs + plan_cus() - 1) / plan_cus()) *
                            (2.5 + (0.08 + 0.0027 * rows + 0.0018 * 32 * nt) * (double)ks_per) +
                        (S > 1 ? 8.0 * S * M * N / 4e6 : 0.0);
       if (best.nt == 0 || t < best_t) {

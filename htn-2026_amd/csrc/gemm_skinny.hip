@@ -240,19 +240,7 @@ bool skinny_nt(const bf16_t* x, int64_t xs, int M, const bf16_t* w, int N, int K
 
 }  // namespace
 
-int skinny_cus() {
-  static int cus = -1;
-  if (cus < 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-      (void)hipGetLastError();
-      n = 0;
-    }
-    cus = n;
-  }
-  return cus;
-}
+int skinny_cus() { return device_cus(); }
 
 // rows per workgroup for N output units over (CU count / S) row blocks: a multiple of 4 (the
 // epilogue's column groups)

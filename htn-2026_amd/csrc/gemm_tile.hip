@@ -532,19 +532,6 @@ bool gemm_tile_ok(int64_t M, int64_t N, int64_t K, int epi, const void* x, int64
   return M * (int64_t)(N / 16) < (1ll << 40) && (M + TM - 1) / TM * tile_nblocks(N, epi) < (1ll << 30);
 }
 
-static int64_t tile_cus() {
-  static int64_t cus = -1;
-  if (cus < 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-      (void)hipGetLastError();
-      n = 256;
-    }
-    cus = n > 0 ? n : 256;
-  }
-  return cus;
-}
 
 // K splits: only the store / residual epilogues split, when the tile grid leaves CUs idle; as
 // many as keep the grid within one workgroup per CU (a grid a little past that puts two on some
@@ -555,7 +542,7 @@ int gemm_tile_splits(int64_t M, int64_t N, int64_t K, int epi) {
   if (epi != EPI_NONE && epi != EPI_RES) return 1;
   const int64_t tiles = (M + TM - 1) / TM * tile_nblocks(N, epi);
   if (tiles >= 160) return 1;
-  int64_t sp = tile_cus() / tiles;
+  int64_t sp = plan_cus() / tiles;
   const int64_t maxsp = (K / TK) / 4;
   if (sp > maxsp) sp = maxsp;
   return sp < 1 ? 1 : (int)sp;
@@ -590,7 +577,7 @@ static bool rows_plan(int64_t M, int64_t N, int64_t K, int epi, bool can_split, 
   if (!QD_TILE_ROWS || M > RW_MAXM || epi == EPI_ARGMAX) return false;
   const bool sw = epi == EPI_SWIGLU;
   if ((sw ? 2 * N : N) * K * 2 >= (1ll << 32)) return false;
-  const int64_t cus = tile_cus(), ksteps = K / TK;
+  const int64_t cus = plan_cus(), ksteps = K / TK;
   // the K split count stays the tiled kernel's (more splits measured slower at 256 rows: qkv in
   // 5 splits 20.2 -> 19.4 us, down in 12 splits 25.5 -> 24.0 us, but their consumers, which
   // read every split's partials, 8.8 -> 12.0 and 5.3 -> 7.7 us)

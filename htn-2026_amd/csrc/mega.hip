@@ -568,19 +568,15 @@ __global__ __launch_bounds__(MG_NT) void mega_step_kernel(MegaParams p) {
 
 // ------------------------------------------------------------------ host side
 int mega_grid() {
-  static int grid = -1;
-  if (grid < 0) {
-    int dev = 0, cus = 0, occ = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, mega_step_kernel, MG_NT, 0) !=
-            hipSuccess) {
+  static const int grid = [] {
+    const int cus = device_cus();
+    int occ = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, mega_step_kernel, MG_NT, 0) != hipSuccess) {
       (void)hipGetLastError();
-      grid = 0;
-    } else {
-      grid = (occ >= 1 && cus >= MIN_WG && cus >= HQ) ? cus : 0;
+      return 0;
     }
-  }
+    return occ >= 1 && cus >= MIN_WG && cus >= HQ ? cus : 0;
+  }();
   return grid;
 }
 

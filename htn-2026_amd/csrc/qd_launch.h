@@ -10,6 +10,23 @@
 enum { EPI_NONE = 0, EPI_RES = 1, EPI_SWIGLU = 2, EPI_ARGMAX = 3 };
 enum { POS_T = 0, POS_SHARED = 1, POS_ROW = 2, POS_TREE = 3, POS_CHUNK = 4 };
 
+// The current device's CU count, asked once (the first caller's device; safe from several threads):
+// 0 if unknown
+inline int device_cus() {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+      (void)hipGetLastError();
+      n = 0;
+    }
+    return n;
+  }();
+  return cus;
+}
+// the count that launch plans divide work by (256, an MI355X's, if unknown)
+inline int64_t plan_cus() { return device_cus() > 0 ? device_cus() : 256; }
+
 // elementwise.hip
 void launch_embed(const int64_t* ids, const bf16_t* table, bf16_t* out, int64_t n, int64_t vocab,
                   int64_t hidden, int64_t out_stride, hipStream_t s);
