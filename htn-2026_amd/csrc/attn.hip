@@ -233,7 +233,6 @@ constexpr int BA_NBUF = QD_BA_NBUF;   // LDS tile buffers (BA_NBUF - 3 tiles in 
 #define QD_BA_TAU 8.0f
 #endif
 constexpr float BA_TAU = QD_BA_TAU;
-constexpr int64_t BA_HALVES_CHUNK = 640;
 constexpr float BA_LN2 = 0.69314718055994531f;
 
 struct BlockAttnLds {
@@ -255,20 +254,20 @@ struct BlockAttnLds {
 //   1 x 8, 300                     26.3 ->  18.2
 // and causal chunks alike (8 x 16, 12000: 142.5 -> 93.7).  A fifth tile buffer (160 KB of LDS)
 // gains nothing: 95.7, 80.0, 46.4, 53.1, 18.2.
-// 33 to 48 tokens (RT = 3, 256 registers; four row tiles would spill) save a quarter of the
-// contraction and pay ~1 us for the combination: 8 x 48, 8000 (splits of 2048 keys) 108.7 ->
-// 96.7, 4 x 40, 8192 (1056) 65.7 -> 62.2, but 1 x 48, 2000 (416) 30.7 -> 31.2 and 8 x 33, 1000
-// (384) 33.5 -> 34.0, so only splits of BA_HALVES_CHUNK keys and more take it.
-template <bool CAUSAL, int RT = 2, bool HALVES = false>
-__global__ __launch_bounds__(512) void block_attn_mfma_kernel(
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
-    const bf16_t* __restrict__ v_cache, const int64_t* __restrict__ base_ptr,
-    const uint64_t* __restrict__ anc, int64_t T, int Hq, int Hkv, int64_t cap, int64_t chunk,
-    float scale_log2, float* ws_acc, float* ws_ml, bf16_t* __restrict__ out) {
+#define QD_BLOCK_PARAMS                                                                         \
+  const bf16_t *__restrict__ q, const bf16_t *__restrict__ k_cache,                             \
+      const bf16_t *__restrict__ v_cache, const int64_t *__restrict__ base_ptr,                 \
+      const uint64_t *__restrict__ anc, int64_t T, int Hq, int Hkv, int64_t cap, int64_t chunk, \
+      float scale_log2, float *ws_acc, float *ws_ml, bf16_t *__restrict__ out
+// One region for every form, at file scope: the kernel below with two of them holds it once, and
+// the compiler sees LDS behind every access (a reference argument cost 1 to 2 %).
+static __shared__ BlockAttnLds sm;
+
+template <bool CAUSAL, int RT, bool HALVES>
+__device__ __forceinline__ void block_attn_block(QD_BLOCK_PARAMS) {
   typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
   typedef __attribute__((ext_vector_type(4))) float f32x4_t;
   constexpr int NH = HALVES ? 2 : 4, NJ = NH / 2;           // 16- and 32-key parts of a wave's tile
-  __shared__ BlockAttnLds sm;
   const int split = blockIdx.x, kvh = blockIdx.y;
   const int splits = gridDim.x;
   const int64_t QB = (T + BA_TQ - 1) / BA_TQ;
@@ -603,6 +602,44 @@ __global__ __launch_bounds__(512) void block_attn_mfma_kernel(
   }
 }
 
+template <bool CAUSAL, int RT = 2, bool HALVES = false>
+__global__ __launch_bounds__(512) void block_attn_mfma_kernel(QD_BLOCK_PARAMS) {
+  block_attn_block<CAUSAL, RT, HALVES>(q, k_cache, v_cache, base_ptr, anc, T, Hq, Hkv, cap, chunk,
+                                       scale_log2, ws_acc, ws_ml, out);
+}
+
+// 17 to 48 tokens: a workgroup takes the half-tile form where its split holds keys enough to pay for
+// it, else the 64-token form: more than 2 tiles of keys up to 32 tokens, more than 7 up to 48 (three
+// row tiles; four would spill).  The keys present decide, not the cache's capacity.  us of the
+// attention alone, sequences x tokens, keys (capacity): 64-token form / half-tile form / here
+//   1 x 17, 64 (32768)     13.7 / 14.8 / 14.3      1 x 33, 100 (32768)    17.8 / 20.5 / 18.3
+//   4 x 32, 256 (8512)     22.7 / 20.9 / 21.0      4 x 33, 100 (8512)     18.8 / 20.8 / 18.4
+//   8 x 32, 8032 (8064)    86.6 / 69.7 / 64.9      1 x 48, 300 (32768)    27.4 / 28.8 / 26.8
+//   4 x 32, 8032 (8512)    53.7 / 46.3 / 44.1      8 x 48, 8048 (8192)    97.4 / 83.8 / 83.3
+constexpr int block_halves_tiles(int rt) { return rt == 3 ? 7 : 2; }
+template <bool CAUSAL, int RT>
+__global__ __launch_bounds__(512) void block_attn_keys_kernel(QD_BLOCK_PARAMS) {
+  const int64_t start = (int64_t)blockIdx.x * chunk, seen = base_ptr[blockIdx.z] + T;
+  int64_t kend = start + chunk < seen ? start + chunk : seen;
+  if (kend > cap) kend = cap;
+  // What the forms have in common is kept apart where that is the faster code (causal, 8 x 48 at
+  // 8000: merged 86.0 us, apart 75.7; 4 x 32 trees there 46.4, 44.1; but 8 x 48 trees at 2000 76.3, 80.5)
+  auto apart = [&]() {
+    if constexpr (CAUSAL || RT == 2)
+      asm volatile("" : "+s"(q), "+s"(k_cache), "+s"(v_cache), "+s"(base_ptr), "+s"(anc));
+  };
+  if (kend - start > BA_KT * block_halves_tiles(RT)) {
+    apart();
+    block_attn_block<CAUSAL, RT, true>(q, k_cache, v_cache, base_ptr, anc, T, Hq, Hkv, cap, chunk,
+                                       scale_log2, ws_acc, ws_ml, out);
+  } else {
+    apart();
+    block_attn_block<CAUSAL, 2, false>(q, k_cache, v_cache, base_ptr, anc, T, Hq, Hkv, cap, chunk,
+                                       scale_log2, ws_acc, ws_ml, out);
+  }
+}
+#undef QD_BLOCK_PARAMS
+
 // the most splits (BLOCK_CHUNK keys each) a launch may use: what the workspace is sized for
 // ------------------------------------------------------------------ decode attention on MFMA (B >= 2)
 // The decode unit (decode_attn_unit: same prologue, same numerics) with its two contractions on
@@ -714,23 +751,24 @@ void launch_block_attn(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_c
   const int64_t chunk = ((cap + use - 1) / use + 31) / 32 * 32;
   const dim3 grid((unsigned)use, (unsigned)Hkv, (unsigned)(B * QB)), block(512);
   const float scale_log2 = (1.0f / sqrtf(128.0f)) * 1.44269504088896341f;
-#define QD_BLOCK(...)                                                                           \
-  block_attn_mfma_kernel<__VA_ARGS__><<<grid, block, 0, s>>>(q, k_cache, v_cache, base, anc, T, Hq, Hkv, \
-                                                             cap, chunk, scale_log2, ws_acc, ws_ml, out)
-  // up to 32 tokens the half-tile form (its comment has both sides measured), up to 48 where a
-  // split is long enough to pay for combining three row tiles
-  if (T <= 16) {
-    if (anc) QD_BLOCK(false, 1, true);
-    else QD_BLOCK(true, 1, true);
-  } else if (T <= 32) {
-    if (anc) QD_BLOCK(false, 2, true);
-    else QD_BLOCK(true, 2, true);
-  } else if (T <= 48 && chunk >= BA_HALVES_CHUNK) {
-    if (anc) QD_BLOCK(false, 3, true);
-    else QD_BLOCK(true, 3, true);
+#define QD_BLOCK(KERNEL, ...)                                                                   \
+  KERNEL<__VA_ARGS__><<<grid, block, 0, s>>>(q, k_cache, v_cache, base, anc, T, Hq, Hkv, cap, chunk, \
+                                             scale_log2, ws_acc, ws_ml, out)
+  // up to 16 tokens the half-tile form (its comment has both sides measured); up to 48 the form that
+  // each workgroup's keys ask for, where a split can hold enough of them
+  const int rt = T <= 16 ? 1 : T <= 32 ? 2 : T <= 48 ? 3 : 4;
+  if (rt == 1) {
+    if (anc) QD_BLOCK(block_attn_mfma_kernel, false, 1, true);
+    else QD_BLOCK(block_attn_mfma_kernel, true, 1, true);
+  } else if (rt == 2 && chunk > BA_KT * block_halves_tiles(2)) {
+    if (anc) QD_BLOCK(block_attn_keys_kernel, false, 2);
+    else QD_BLOCK(block_attn_keys_kernel, true, 2);
+  } else if (rt == 3 && chunk > BA_KT * block_halves_tiles(3)) {
+    if (anc) QD_BLOCK(block_attn_keys_kernel, false, 3);
+    else QD_BLOCK(block_attn_keys_kernel, true, 3);
   } else {
-    if (anc) QD_BLOCK(false);
-    else QD_BLOCK(true);
+    if (anc) QD_BLOCK(block_attn_mfma_kernel, false);
+    else QD_BLOCK(block_attn_mfma_kernel, true);
   }
 #undef QD_BLOCK
   if (use > 1)      // one split writes its rows itself

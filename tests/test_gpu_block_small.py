@@ -54,3 +54,12 @@ def test_small_blocks(B, base, spare, T, tree):
             bound = 2.0 ** -8 * (p @ vv.abs()) + bf16_ulp(want.float()).double()
             d = (got[:, :, 4 * h + i].double() - want).abs()
             assert bool((d <= bound).all()), f"head {4 * h + i}: {float((d - bound).max())}"
+
+
+# a cache with room for much more than it holds, and keys on both sides of the counts (2 and 7 tiles of
+# 64) from which a workgroup's split takes the half-tile form: 17..48 tokens
+@pytest.mark.parametrize("tree", [True, False])
+@pytest.mark.parametrize("T", [17, 32, 33, 48])
+@pytest.mark.parametrize("keys", [60, 128, 129, 448, 449, 513, 1100])
+def test_form_by_keys(keys, T, tree):
+    test_small_blocks(2, keys - T, 4096 - keys, T, tree)
