@@ -50,8 +50,8 @@ constexpr int TK = 64;                         // K per stage: 128 bytes of ever
 
 // WAIT: the 8 wait states that a VALU read of the result needs, in the same asm.  The compiler does
 // not see the latency of an MFMA in asm and may copy an accumulator right behind one (it does where
-// the main loop's accumulators become the tail's), so the last MFMA of a K half carries them; the
-// others are followed by an MFMA and the rest of that wait.
+// the main loop's accumulators become the tail's), so the last MFMA of a stage carries them, and of
+// each half in the tail; the others are followed by an MFMA and the rest of that wait.
 template <bool WAIT>
 __device__ __forceinline__ void mfma_acc(f32x4_t& acc, uint4 a, uint4 b) {
   if constexpr (WAIT)
@@ -189,15 +189,16 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
       f.v[t] = sm[px + 128 * (t - NT) + u];
     }
   };
-  // contract the half in cur; RD: read half (rb, hf) into nxt; LD: load stage st into buffer lb
-#define QD_HALF(LD, RD, cur, nxt, rb, hf, st, lb)                                              \
+  // contract the half in cur; RD: read half (rb, hf) into nxt; LD: load stage st into buffer lb;
+  // WT: the last MFMA carries its wait
+#define QD_HALF(WT, LD, RD, cur, nxt, rb, hf, st, lb)                                          \
   _Pragma("unroll") for (int g_ = 0; g_ < PER; ++g_) {                                         \
     if (LD) load(st, lb, g_);                                                                  \
     if (RD) rd(nxt, rb, hf, g_);                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                         \
     _Pragma("unroll") for (int e_ = g_ * MT * NT / PER; e_ < (g_ + 1) * MT * NT / PER; ++e_) { \
       if (e_ + 1 < MT * NT) mfma_acc<false>(acc[e_ % NT][e_ / NT], cur.v[e_ % NT], cur.v[NT + e_ / NT]); \
-      else mfma_acc<true>(acc[e_ % NT][e_ / NT], cur.v[e_ % NT], cur.v[NT + e_ / NT]);         \
+      else mfma_acc<WT>(acc[e_ % NT][e_ / NT], cur.v[e_ % NT], cur.v[NT + e_ / NT]);           \
     }                                                                                          \
     __builtin_amdgcn_sched_barrier(0);                                                         \
   }
@@ -219,27 +220,27 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
   // visible and stage s's buffer free.
   int b = 0, s = 0;
   for (; s + NBUF < stages; ++s) {
-    QD_HALF(false, true, f0, f1, b, 1, 0, 0);
+    QD_HALF(false, false, true, f0, f1, b, 1, 0, 0);
     if (toucher) wait_vm<PER * (NBUF - 2) + NBUF - 1>();
     else wait_vm<PER * (NBUF - 2)>();
     lds_barrier();
     const int bn = b + 1 < NBUF ? b + 1 : 0;
-    QD_HALF(true, true, f1, f0, bn, 0, s + NBUF, b);
+    QD_HALF(true, true, true, f1, f0, bn, 0, s + NBUF, b);
     if (toucher) touch(s + NBUF + TOUCH);
     b = bn;
   }
   settle();
   for (; s + 1 < stages; ++s) {                // the last stages: nothing left to load
-    QD_HALF(false, true, f0, f1, b, 1, 0, 0);
+    QD_HALF(true, false, true, f0, f1, b, 1, 0, 0);
     wait_stages<PER, NBUF - 2>(stages - 2 - s);
     lds_barrier();
     const int bn = b + 1 < NBUF ? b + 1 : 0;
-    QD_HALF(false, true, f1, f0, bn, 0, 0, 0);
+    QD_HALF(true, false, true, f1, f0, bn, 0, 0, 0);
     settle();
     b = bn;
   }
-  QD_HALF(false, true, f0, f1, b, 1, 0, 0);
-  QD_HALF(false, false, f1, f0, b, 0, 0, 0);
+  QD_HALF(true, false, true, f0, f1, b, 1, 0, 0);
+  QD_HALF(true, false, false, f1, f0, b, 0, 0, 0);
 #undef QD_HALF
   wait_vm<0>();                                // no load outlives the workgroup
   settle();
