@@ -392,10 +392,14 @@ constexpr bool quad_fits() {
 static_assert(quad_fits(), "the CU's LDS");
 
 
+// Split launches take one of the first two: their splits times 128 x 128 tiles are at most the CUs
+// (gemm_tile_splits), one round of {4, 4}.
+constexpr int QUAD_SPLIT = 2;
+
 int quad_plan(int64_t M, int64_t N, bool sw, int64_t splits, int64_t stages) {
   int best = -1;
   double best_t = 0;
-  for (int i = 0; i < QUADS; ++i) {
+  for (int i = 0; i < (splits > 1 ? QUAD_SPLIT : QUADS); ++i) {
     const QuadShape& q = QUAD[i];
     if (sw && q.nt % 2) continue;
     const int64_t bm = 32 * q.mt, bn = quad_outs(q.nt, sw);
@@ -426,7 +430,7 @@ template <int EPI, bool SPLIT, int I = 0>
 void quad_pick(int i, const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
                bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int splits, int ks_per,
                int wide, float* part, hipStream_t s) {
-  if constexpr (I < QUADS) {
+  if constexpr (I < (SPLIT ? QUAD_SPLIT : QUADS)) {
     if constexpr (EPI != EPI_SWIGLU || QUAD[I].nt % 2 == 0) {
       if (i == I)
         return quad_go<I, EPI, SPLIT>(x, xs, M, w, N, K, out, os, res, rs, splits, ks_per, wide, part, s);
@@ -512,19 +516,22 @@ static SmallPlan quad_small_plan(int64_t M, int64_t N, int64_t K, bool sw, int64
   return best;
 }
 
+constexpr int quad_small_nbuf(int nt) { return nt == 2 || nt == 6 ? 4 : 3; }
+
 template <int EPI, bool SPLIT>
 static void quad_small_go(const SmallPlan& P, const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w,
                           int64_t N, int64_t K, bf16_t* out, int64_t os, const bf16_t* res,
                           int64_t rs, int wide, float* part, hipStream_t s) {
   const int64_t mbl = (M + 63) / 64, nbl = (N + P.outs - 1) / P.outs;
-#define QD_SMALL(NT, NB)                                                                        \
-  gemm_quad_kernel<EPI, SPLIT, 2, NT, NB><<<dim3((unsigned)(mbl * nbl * P.splits)), dim3(256), 0, s>>>( \
+#define QD_SMALL(NT)                                                                            \
+  gemm_quad_kernel<EPI, SPLIT, 2, NT, quad_small_nbuf(NT)><<<dim3((unsigned)(mbl * nbl * P.splits)), dim3(256), \
+                                                             0, s>>>(                           \
       x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, P.outs, P.ks_per, out, os, res, rs, wide, part, \
       nullptr, nullptr, nullptr)
-  if (P.nt == 2) QD_SMALL(2, 4);
-  else if (P.nt == 4) QD_SMALL(4, 3);
-  else if (P.nt == 6) QD_SMALL(6, 4);
-  else if constexpr (EPI != EPI_SWIGLU) QD_SMALL(3, 3);
+  if (P.nt == 2) QD_SMALL(2);
+  else if (P.nt == 4) QD_SMALL(4);
+  else if (P.nt == 6) QD_SMALL(6);
+  else if constexpr (EPI != EPI_SWIGLU) QD_SMALL(3);
 #undef QD_SMALL
 }
 
@@ -556,6 +563,21 @@ int launch_quad_small(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, i
   else if (epi == EPI_SWIGLU) quad_small_go<EPI_SWIGLU, false>(P, x, xs, M, w, N, K, out, os, res, rs, wide, part, s);
   else quad_small_go<EPI_NONE, false>(P, x, xs, M, w, N, K, out, os, res, rs, wide, part, s);
   return 0;
+}
+
+// What the launchers above run, for qd_gemm_quad_plan: out = MT, NT, stage buffers, K splits, stages per
+// split, output columns per workgroup.
+void quad_query(int64_t M, int64_t N, int64_t K, int epi, int splits, int ks_per, int64_t* out) {
+  const bool sw = epi == EPI_SWIGLU;
+  const QuadShape& q = QUAD[quad_plan(M, N, sw, splits, ks_per)];
+  const int64_t v[6] = {q.mt, q.nt, q.nbuf, splits, ks_per, quad_outs(q.nt, sw)};
+  for (int i = 0; i < 6; ++i) out[i] = v[i];
+}
+
+void quad_small_query(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats, int64_t* out) {
+  const SmallPlan P = quad_small_plan(M, N, K, epi == EPI_SWIGLU, part_floats / (M * N));
+  const int64_t v[6] = {2, P.nt, quad_small_nbuf(P.nt), P.splits, P.ks_per, P.outs};
+  for (int i = 0; i < 6; ++i) out[i] = v[i];
 }
 
 // split partials the two above can use at most

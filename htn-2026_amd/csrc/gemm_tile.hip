@@ -758,6 +758,31 @@ int gemm_tile_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
   return splits;
 }
 
+// K splits of a launch that reduces them itself, and stages per split
+static int tile_launch_splits(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats, int& ks_per) {
+  // from 1024 rows on, whole 256-column blocks are not split (the largest tiles fill the chip)
+  int splits = M >= 1024 && N % 256 == 0 ? 1 : gemm_tile_splits(M, N, K, epi);
+  if (splits > 1 && part_floats < (int64_t)splits * M * N) splits = 1;
+  const int ksteps = (int)(K / TK);
+  ks_per = (ksteps + splits - 1) / splits;
+  return (ksteps + ks_per - 1) / ks_per;                // no empty split
+}
+
+int gemm_quad_query(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats, int64_t* out) {
+  const void* a = reinterpret_cast<const void*>(256);
+  RowsPlan P;
+  if (M < GEMM_SMALL_MIN_M || !gemm_tile_ok(M, N, K, epi, a, K, a, a, N, a, N)) return 0;
+  if (M < GEMM_TILE_MIN_M) {
+    quad_small_query(M, N, K, epi, part_floats, out);
+    return 1;
+  }
+  if (rows_launch_plan(M, N, K, epi, false, part_floats, P) == 1) return 0;
+  int ks_per;
+  const int splits = tile_launch_splits(M, N, K, epi, part_floats, ks_per);
+  quad_query(M, N, K, epi, splits, ks_per, out);
+  return 1;
+}
+
 // Returns the number of argmax partials per row written (EPI_ARGMAX), else 0.
 int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,
                          int64_t K, bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi,
@@ -797,12 +822,8 @@ int64_t launch_gemm_tile(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w
     return 0;
   }
   const int64_t mblocks = (M + TM - 1) / TM, nblocks = tile_nblocks(N, epi);
-  // from 1024 rows on, whole 256-column blocks are not split (the largest tiles fill the chip)
-  int splits = M >= 1024 && N % 256 == 0 ? 1 : gemm_tile_splits(M, N, K, epi);
-  if (splits > 1 && (!part || part_floats < (int64_t)splits * M * N)) splits = 1;
-  const int ksteps = (int)(K / TK);
-  const int ks_per = (ksteps + splits - 1) / splits;
-  splits = (ksteps + ks_per - 1) / ks_per;              // no empty split
+  int ks_per;
+  const int splits = tile_launch_splits(M, N, K, epi, part ? part_floats : 0, ks_per);
   // the four-wave kernel; the 128 x 128 tiles below where its 32-bit offsets do not reach, and
   // for the LM head's 65..128 rows
   const bool quad = epi != EPI_ARGMAX &&

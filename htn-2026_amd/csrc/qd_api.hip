@@ -768,6 +768,11 @@ int qd_gemm_rows_plan(int64_t M, int64_t N, int64_t K, int32_t epi, int64_t part
   return gemm_rows_query(M, N, K, epi, partials_only != 0, part_floats, out);
 }
 
+int qd_gemm_quad_plan(int64_t M, int64_t N, int64_t K, int32_t epi, int64_t part_floats, int64_t* out) {
+  if (!out || M <= 0 || N <= 0 || K <= 0 || part_floats < 0 || epi < EPI_NONE || epi > EPI_SWIGLU) return QD_EARG;
+  return gemm_quad_query(M, N, K, epi, part_floats, out);
+}
+
 // ------------------------------------------------------------------ graphs
 int qd_graph_begin(void* stream) {
   if (!stream) return QD_EARG;  // the legacy null stream cannot be captured

@@ -111,6 +111,9 @@ int gemm_tile_splits(int64_t M, int64_t N, int64_t K, int epi);
 // tiles per wave, activation halves, K splits, K steps per split, grid, static LDS bytes.
 int gemm_rows_query(int64_t M, int64_t N, int64_t K, int epi, bool partials_only,
                     int64_t part_floats, int64_t* out);
+// The four-wave kernel's launch (qd_gemm_quad_plan): 0 where launch_gemm_tile takes another kernel, else
+// 1 with out[6] as quad_query
+int gemm_quad_query(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats, int64_t* out);
 int64_t gemm_tile_ws_floats(int64_t M, int64_t N, int64_t K, int epi);
 // the most it asks for over B t rows, 1 <= t <= T
 int64_t gemm_tile_ws_floats_upto(int64_t B, int64_t T, int64_t N, int64_t K, int epi);
@@ -129,6 +132,8 @@ int launch_quad_small(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, i
                       bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi, float* part,
                       int64_t part_floats, hipStream_t s);
 int64_t quad_small_ws_floats(int64_t M, int64_t N, int64_t K);
+void quad_query(int64_t M, int64_t N, int64_t K, int epi, int splits, int ks_per, int64_t* out);
+void quad_small_query(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats, int64_t* out);
 int64_t launch_lm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
                        float* pval, int32_t* pidx, float* logits, hipStream_t s);
 // rows from which the four-wave kernel's small plan takes over (M <= 32: the skinny kernel)

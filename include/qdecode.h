@@ -273,6 +273,11 @@ int qd_block_step(const qd_weights *w, const qd_block_state *st, void *stream);
 int qd_gemm_rows_plan(int64_t M, int64_t N, int64_t K, int32_t epi, int64_t part_floats,
                       int32_t partials_only, int64_t *out);
 
+/* The same for the four-wave GEMM (33..64 rows, 257 and more; contiguous rows, 16-byte aligned
+ * operands): 1 with out[6] = {activation tiles, weight tiles of a wave, stage buffers, K splits, K steps
+ * per split, output columns per workgroup}, 0 when another kernel serves the shape. */
+int qd_gemm_quad_plan(int64_t M, int64_t N, int64_t K, int32_t epi, int64_t part_floats, int64_t *out);
+
 /* hipGraph capture of whatever is enqueued on `stream` between begin and end (replaces the
  * torch.cuda.CUDAGraph capture of the decode step, engine/engine.py:685-713). */
 int qd_graph_begin(void *stream);

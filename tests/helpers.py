@@ -167,3 +167,31 @@ def engine_step_logits(eng, prompt, N):
     sh.decode.check()
     return (emitted.T.cpu().numpy(), arg.T.cpu().numpy(),
             logits.transpose(0, 1).contiguous().cpu())
+
+
+def check_linear(ops, epi, x, N, g, **kw):
+    """GPU: ops.linear over the rows x with random weights (generator g), every output within the
+    roundings of its epilogue around the fp64 product."""
+    bf = torch.bfloat16
+    rnd = lambda *s, std: torch.empty(s, dtype=bf, device="cuda").normal_(0, std, generator=g)  # noqa: E731
+    w = rnd(2 * N if epi == ops.EPI_SWIGLU else N, x.shape[1], std=0.05)
+    res = rnd(x.shape[0], N, std=2.0)
+    got = ops.linear(x, w, epi, res=res if epi == ops.EPI_RES else None, **kw).float()
+    a = (x.double() @ w.double().t()).to(bf).float()
+    if epi == ops.EPI_SWIGLU:
+        # one ulp in bf16(gate), bf16(up) and bf16(silu) each, propagated, and two of the output
+        gate, up = a[:, :N], a[:, N:]
+        sg = torch.sigmoid(gate)
+        s = (gate * sg).to(bf).float()
+        want = (s * up).to(bf).float()
+        bound = (up.abs() * ((sg * (1 + gate * (1 - sg))).abs() * bf16_ulp(gate) + bf16_ulp(s))
+                 + s.abs() * bf16_ulp(up) + 2 * bf16_ulp(torch.maximum(got.abs(), want.abs())) + 2 ** -12)
+    elif epi == ops.EPI_RES:
+        # one ulp of bf16(a) may survive cancellation into the sum
+        want = (res.float() + a).to(bf).float()
+        bound = bf16_ulp(a) + 2 * bf16_ulp(torch.maximum(got.abs(), want.abs()))
+    else:
+        want = a
+        bound = 2 * bf16_ulp(torch.maximum(got.abs(), want.abs())) + 2 ** -9
+    d = (got - want).abs()
+    assert bool((d <= bound).all()), f"max excess {float((d - bound).max())}"

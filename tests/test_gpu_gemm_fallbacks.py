@@ -1,10 +1,10 @@
 """The GEMM kernels behind the usual ones, against fp64 products: activation rows too far apart for
-32-bit offsets."""
+32-bit offsets, and at 33 to 64 rows the widths and alignments that the four-wave kernel does not take."""
 
 import pytest
 import torch
 
-from helpers import bf16_ulp
+from helpers import check_linear
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
@@ -14,34 +14,6 @@ BF = torch.bfloat16
 def ops():
     from qdecode import ops as o
     return o
-
-
-def _rnd(g, *s, std=1.0):
-    return torch.empty(s, dtype=BF, device="cuda").normal_(0, std, generator=g)
-
-
-def _check(ops, epi, x, N, g, **kw):
-    """ops.linear over x with random weights, each output within the roundings of its epilogue."""
-    K = x.shape[1]
-    w, res = _rnd(g, 2 * N if epi == ops.EPI_SWIGLU else N, K, std=0.05), _rnd(g, x.shape[0], N, std=2.0)
-    got = ops.linear(x, w, epi, res=res if epi == ops.EPI_RES else None, **kw).float()
-    a = (x.double() @ w.double().t()).to(BF).float()
-    if epi == ops.EPI_SWIGLU:
-        # one ulp in bf16(gate), bf16(up) and bf16(silu) each, propagated, and two of the output
-        gate, up = a[:, :N], a[:, N:]
-        sg = torch.sigmoid(gate)
-        s = (gate * sg).to(BF).float()
-        want = (s * up).to(BF).float()
-        bound = (up.abs() * ((sg * (1 + gate * (1 - sg))).abs() * bf16_ulp(gate) + bf16_ulp(s))
-                 + s.abs() * bf16_ulp(up) + 2 * bf16_ulp(torch.maximum(got.abs(), want.abs())) + 2 ** -12)
-    elif epi == ops.EPI_RES:
-        want = (res.float() + a).to(BF).float()
-        bound = bf16_ulp(a) + 2 * bf16_ulp(torch.maximum(got.abs(), want.abs()))
-    else:
-        want = a
-        bound = 2 * bf16_ulp(torch.maximum(got.abs(), want.abs())) + 2 ** -9
-    d = (got - want).abs()
-    assert bool((d <= bound).all()), f"max excess {float((d - bound).max())}"
 
 
 # the skinny kernel's buffer extent (32 rows), the four-wave kernel's offsets (33 and 300 rows, in
@@ -55,6 +27,32 @@ def test_long_row_strides(ops, M, stride, epi):
     g.manual_seed(M + epi)
     K = 1024
     x = torch.empty((M - 1) * stride + K, dtype=BF, device="cuda").as_strided((M, K), (stride, 1))
-    x.copy_(_rnd(g, M, K))
-    _check(ops, epi, x, 512, g)                  # its workspace: K splits where the plan has them
-    _check(ops, epi, x, 512, g, ws=torch.zeros(256, dtype=torch.uint8, device="cuda"))
+    x.normal_(0, 1, generator=g)
+    check_linear(ops, epi, x, 512, g)                  # its workspace: K splits where the plan has them
+    check_linear(ops, epi, x, 512, g, ws=torch.zeros(256, dtype=torch.uint8, device="cuda"))
+
+
+# N is not a multiple of 128 (SwiGLU: 64): the LDS-staged kernel (K a multiple of 512) and the plain
+# one, at odd widths too
+@pytest.mark.parametrize("epi", [0, 1, 2])
+@pytest.mark.parametrize("N,K", [(192, 1024), (96, 512), (72, 512), (161, 1024), (192, 640), (96, 128)])
+@pytest.mark.parametrize("M", [33, 48, 64])
+def test_widths_at_33_to_64_rows(ops, M, N, K, epi):
+    if epi == ops.EPI_SWIGLU and N % 64 == 0:
+        N += 32
+    print(f"\n[case] {M} x {N} x {K}, epilogue {epi}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K + epi)
+    x = torch.empty((M, K), dtype=BF, device="cuda").normal_(0, 1, generator=g)
+    check_linear(ops, epi, x, N, g)
+
+
+@pytest.mark.parametrize("M", [33, 64])
+def test_unaligned_output_at_33_to_64_rows(ops, M):
+    """Output rows that start 2 bytes off: not the four-wave kernel's 8-byte stores."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    x = torch.empty((M, 1024), dtype=BF, device="cuda").normal_(0, 1, generator=g)
+    buf = torch.full((M, 260), 7.0, dtype=BF, device="cuda")
+    check_linear(ops, 0, x, 256, g, out=buf[:, 1:257])
+    assert bool((buf[:, :1] == 7).all()) and bool((buf[:, 257:] == 7).all())

@@ -1,5 +1,6 @@
-"""The four-wave GEMM of 257 and more rows (gemm_quad.hip): every tile shape its plan picks for the
-model's projections, ragged row counts around the tiles, and outputs that are only 8-byte aligned.
+"""The four-wave GEMM (gemm_quad.hip): every tile shape its plan picks for the model's projections,
+every compiled instance, ragged row counts around the tiles, and outputs that are only 8-byte
+aligned.  (tests/test_quad_plan.py checks that the shapes here cover what the plan picks.)
 
 An output's accumulation runs through K in order whatever the tile, so unsplit launches agree bit
 for bit on the rows they share; the largest launch is held to an fp64 product."""
@@ -7,14 +8,33 @@ for bit on the rows they share; the largest launch is held to an fp64 product.""
 import pytest
 import torch
 
-from helpers import bf16_ulp
+from helpers import bf16_ulp, check_linear
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
 SHAPES = {"qkv": (6144, 2560), "o": (2560, 4096), "gu": (9728, 2560), "down": (2560, 9728)}
-# between them these counts take all 13 tile shapes; 257, 1025 and 2049 leave one row in the last
-# row block, 1023 and 4095 fill all but one
-ROWS = [257, 300, 399, 513, 601, 768, 1023, 1025, 1500, 2049, 3000, 4095, 6001]
+# between them these counts take every tile shape that the plan picks for 257 to 16384 rows of these
+# projections, with each epilogue that picks it; 257, 1025 and 2049 leave one row in the last row
+# block, 1023 and 4095 fill all but one
+ROWS = [257, 300, 399, 513, 601, 768, 800, 1023, 1025, 1200, 1500, 1600, 2049, 2600, 3000, 3100, 3300,
+        4095, 4500, 6001]
+# one launch of every compiled instance, ten K stages and more: (split, MT, NT) -> rows, outputs, K, for
+# each epilogue that it is compiled for (split partials: one instance serves all)
+INSTANCES = {
+    ("split", 2, 2): (33, 128, 640), ("split", 2, 3): (33, 6144, 2560), ("split", 2, 4): (33, 4096, 9728),
+    ("split", 2, 6): (33, 9728, 9728), ("split", 4, 3): (257, 128, 640), ("split", 4, 4): (385, 128, 9728),
+    ("plain", 2, 2): (63, 4096, 640), ("plain", 2, 3): (33, 20480, 640), ("plain", 2, 4): (33, 30720, 640),
+    ("plain", 2, 6): (33, 45056, 640), ("plain", 4, 3): (1025, 256, 640), ("plain", 4, 4): (257, 9728, 640),
+    ("plain", 4, 5): (385, 9728, 640), ("plain", 4, 6): (8193, 512, 640), ("plain", 4, 8): (3073, 2560, 640),
+    ("plain", 4, 10): (3073, 3072, 1152), ("plain", 6, 5): (8193, 640, 640),
+    ("plain", 6, 6): (769, 9728, 1152), ("plain", 6, 8): (2817, 4096, 640), ("plain", 8, 4): (6913, 1024, 640),
+    ("plain", 8, 5): (769, 9728, 640), ("plain", 8, 6): (3073, 3072, 640), ("plain", 8, 8): (4865, 2560, 640),
+    ("swiglu", 2, 2): (33, 128, 640), ("swiglu", 2, 4): (33, 9728, 640), ("swiglu", 2, 6): (33, 20480, 640),
+    ("swiglu", 4, 4): (257, 128, 640), ("swiglu", 4, 6): (257, 6144, 640), ("swiglu", 4, 8): (257, 9728, 640),
+    ("swiglu", 4, 10): (385, 9728, 640), ("swiglu", 6, 6): (1537, 2560, 640),
+    ("swiglu", 6, 8): (513, 9728, 640), ("swiglu", 8, 4): (641, 4096, 640), ("swiglu", 8, 6): (8193, 512, 640),
+    ("swiglu", 8, 8): (577, 9728, 640),
+}
 
 
 @pytest.fixture(scope="module")
@@ -79,8 +99,8 @@ def test_split_launches(ops, name, M):
     assert bool(((got - want).abs() <= bound).all())
 
 
-# 33..64 rows: one row block of 64, blocks of 40 to 96 columns, 1 to 8 K splits as the plan and the
-# partial room decide (none: unsplit)
+# 33..64 rows: one row block of 64, 40 to 96 columns per workgroup and 1 to 8 K splits as the plan
+# decides; without room for partials unsplit, in blocks of 16 to 40 columns
 @pytest.mark.parametrize("name", list(SHAPES))
 @pytest.mark.parametrize("M", [33, 47, 64])
 def test_small_row_counts(ops, name, M):
@@ -121,6 +141,17 @@ def test_outputs_aligned_to_8_bytes(ops, name, M):
     _linear(ops, name, x, w, r2, out=out)
     assert torch.equal(out, want)
     assert bool((buf[:, :4] == 7).all()) and bool((buf[:, 4 + N:] == 7).all())
+
+
+@pytest.mark.parametrize("kind,mt,nt", list(INSTANCES))
+def test_every_instance(ops, kind, mt, nt):
+    M, N, K = INSTANCES[kind, mt, nt]
+    print(f"\n[case] {kind} {{{mt}, {nt}}}: {M} x {N} x {K}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K)
+    x = torch.empty((M, K), dtype=BF, device="cuda").normal_(0, 1, generator=g)
+    for epi in (ops.EPI_SWIGLU,) if kind == "swiglu" else (ops.EPI_NONE, ops.EPI_RES):
+        check_linear(ops, epi, x, N, g)
 
 
 @pytest.mark.parametrize("B,S,N", [(33, 20, 4), (48, 40, 4), (100, 12, 3), (130, 9, 3)])
