@@ -585,7 +585,8 @@ static int64_t gemm_mt(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
       const int64_t parts = launch_lm_quad(x, xs, M, w, N, K, pval, pidx, logits, s);
       if (parts > 0) return parts;
     }
-    if (M <= 64 && K % 512 == 0 && aligned && P >= 1) {
+    // (one partial per workgroup and row: the workspace has room for min(N, 1024) of them)
+    if (M <= 64 && K % 512 == 0 && aligned && P >= 1 && P <= 1024 && N >= P) {
       if (M <= 16) return stream_mt<1, EPI>(x, xs, M, w, N, K, out, os, res, rs, pval, pidx, logits, P, s);
       if (M <= 32) return stream_mt<2, EPI>(x, xs, M, w, N, K, out, os, res, rs, pval, pidx, logits, P, s);
       return stream_mt<4, EPI>(x, xs, M, w, N, K, out, os, res, rs, pval, pidx, logits, P, s);

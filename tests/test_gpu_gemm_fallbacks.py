@@ -1,5 +1,6 @@
 """The GEMM kernels behind the usual ones, against fp64 products: activation rows too far apart for
-32-bit offsets, and at 33 to 64 rows the widths and alignments that the four-wave kernel does not take."""
+32-bit offsets, and at 33 to 64 rows the widths, alignments and vocabularies that the four-wave kernel does
+not take."""
 
 import pytest
 import torch
@@ -56,3 +57,21 @@ def test_unaligned_output_at_33_to_64_rows(ops, M):
     buf = torch.full((M, 260), 7.0, dtype=BF, device="cuda")
     check_linear(ops, 0, x, 256, g, out=buf[:, 1:257])
     assert bool((buf[:, :1] == 7).all()) and bool((buf[:, 257:] == 7).all())
+
+
+# a vocabulary that is no multiple of 4, or under 256: the weight-streaming kernel (K a multiple of 512)
+# and the LDS-staged and plain ones
+@pytest.mark.parametrize("V,K", [(50257, 1024), (4099, 2560), (250, 512), (1001, 640), (37, 256)])
+@pytest.mark.parametrize("M", [33, 48, 64])
+def test_lm_head_vocabularies_at_33_to_64_rows(ops, M, V, K):
+    print(f"\n[case] lm_head_argmax {M} rows, vocabulary {V}, K {K}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + V)
+    rnd = lambda *s, std: torch.empty(s, dtype=BF, device="cuda").normal_(0, std, generator=g)  # noqa: E731
+    x, w, nw = rnd(M, K, std=1.0), rnd(V, K, std=0.02), rnd(K, std=0.1) + 1
+    logits = torch.empty((M, V), dtype=torch.float32, device="cuda")
+    tok = ops.lm_head_argmax(x, w, nw, 1e-6, logits=logits)
+    # against the kernel's own normalised rows the logits carry fp32 accumulation error only
+    want = ops.rmsnorm(x, nw, 1e-6).double() @ w.double().t()
+    assert float((logits.double() - want).abs().max()) <= 1e-4
+    assert torch.equal(tok.cpu(), torch.argmax(logits.to(BF).float().cpu(), dim=-1))
