@@ -181,11 +181,10 @@ SHAPES = {"qkv": (6144, 2560), "o": (2560, 4096), "gu": (9728, 2560), "down": (2
 
 
 # 1..2 rows: vector GEMV; 3..32: the skinny kernel (one workgroup per CU; 20 rows: a ragged
-# second activation tile); 64: the LDS-staged MFMA kernel; 100, 256, 600 rows: the LDS-tiled
-# kernel (128-row tiles with a ragged last tile; K split over workgroups with the fp32 partials
-# summed by a second kernel where the tile grid is small: qkv / o / down at 100 and 256 rows,
-# o / down at 600); 1040 rows: the 256 x 256-tile prefill kernel (four full row blocks and a
-# ragged 16-row one)
+# second activation tile); 64: the four-wave kernel's one row block; 65, 100, 200, 256: the all-rows
+# kernel; 600 and 1040 rows: the four-wave kernel with ragged last row blocks.  K is split over
+# workgroups, with the fp32 partials summed by a second kernel, where the grid is small: qkv / o / down
+# from 64 to 256 rows, o / down at 600
 @pytest.mark.parametrize("B", [1, 2, 3, 16, 20, 32, 64, 65, 100, 200, 256, 600, 1040])
 @pytest.mark.parametrize("name", ["qkv", "o", "gu", "down"])
 def test_linear_epilogues(ops, name, B):
@@ -247,8 +246,8 @@ def test_linear_epilogues(ops, name, B):
         assert bool((d <= bound).all()), f"{name}: max excess {float((d - bound).max())}"
 
 
-# Ragged shapes across every dispatch range (vector GEMV, skinny MFMA, LDS-staged, all-rows with
-# and without K splits and activation halves, 128 x 128 and 256 x 256 tiles): seeded random
+# Ragged shapes across every dispatch range (vector GEMV, skinny MFMA, all-rows with and without K
+# splits and activation halves, four-wave at 33 to 64 and from 257 rows): seeded random
 # (rows, outputs, K, epilogue), against fp64 with test_linear_epilogues' bounds
 _RNG = np.random.default_rng(2024)
 RAGGED = [(int(_RNG.integers(1, 65) if i % 2 else _RNG.integers(65, 1101)),
@@ -298,14 +297,14 @@ def test_linear_ragged_shapes(ops, M, N, K, epi):
         assert bool((d <= bound).all()), f"gate/up: max excess {float((d - bound).max())}"
 
 
-# The 256 x 256-tile kernel's shortest pipelines (K = 128: its two K stages both loaded up front;
-# K = 384: six) with a ragged last row block: plain against fp64, residual in place, and SwiGLU
+# The four-wave kernel's shortest pipelines from 1024 rows (K = 128: its two K stages both loaded up
+# front; K = 384: six) with a ragged last row block: plain against fp64, residual in place, and SwiGLU
 # bit for bit against the oracle's SwiGLU of the same kernel's own gate and up projections (the
 # gate / up rows reach it through the 64-deep stages' row mapping)
 @pytest.mark.parametrize("K", [128, 384])
 def test_big_tile_short_k(ops, K):
     M, N = 1100, 512
-    say(f"256 x 256 tiles: M={M} N={N} K={K}")
+    say(f"four-wave kernel, short K: M={M} N={N} K={K}")
     g = torch.Generator().manual_seed(77 + K)
     x = rnd(g, M, K)
     w = rnd(g, 2 * N, K, scale=0.05)
@@ -331,9 +330,9 @@ def test_big_tile_short_k(ops, K):
 
 
 # ------------------------------------------------------------------ LM head + argmax
-# 1-2 rows: the vector kernel; 3-64: the weight-streaming MFMA kernel (16 / 32 / 64-row
-# activation tiles); 72: the 128 x 128 tiled kernel; 160, 256: the 256 x 256 tile with the argmax
-# epilogue (one partly filled / one full row block, and the vocabulary's last block half full)
+# 1-2 rows: the vector kernel; 8, 24: the skinny argmax kernel (16 / 32-row activation tiles); 40, 160,
+# 256: the four-wave kernel with the argmax epilogue (64-row and 256-row blocks, partly filled and
+# full, and the vocabulary's last block partly full); 72: the 128 x 128 tiled kernel
 @pytest.mark.parametrize("B", [1, 2, 8, 24, 40, 72, 160, 256])
 def test_lm_head_argmax(ops, B):
     say(f"lm_head_argmax B={B}")
