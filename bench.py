@@ -22,7 +22,7 @@ Workloads (the benchmark's configurations 2-5; configuration 1 is the CPU parity
          (where bandwidth, not launch latency, binds): GB/s, fraction of 8 TB/s, and a device
          copy of the same bytes as the read+write yardstick.
   prefill_gemm  the four projections of a prefill chunk (32768 rows, the engine's chunk) through
-         qd_linear (the 256 x 256-tile MFMA kernel) and, beside them, torch.matmul (hipBLASLt)
+         qd_linear (the four-wave MFMA kernel) and, beside them, torch.matmul (hipBLASLt)
          on the same operands: us per launch and TFLOP/s against the 2.5 PFLOP/s bf16 dense peak.
   step_ms  per-step spread (median, p90, min, max) of the same K steps replayed again with an
          event after each step (the headline timing has no events between steps).

@@ -213,11 +213,9 @@ constexpr int64_t BLOCK_CHUNK = 512;
 //    receives element b of the 8-byte pieces that lanes a, a + 4, a + 8, a + 12 address, so lane
 //    i addressing dims 16 dt + 4 (i % 4) .. + 3 of key 4q + i / 4 makes lane c receive
 //    V[4q + r][16 dt + c], r = 0..3 (measured on MI355X with an in-bounds layout probe);
-//  * pipeline: three LDS tile buffers; in the step of tile i a wave contracts S' of tile i + 1
-//    (its MFMAs independent of the softmax of tile i, which the compiler interleaves with them),
-//    runs the softmax and O update of tile i, and the workgroup stages tile i + 2 from registers
-//    loaded two steps earlier (thread i moves K and V unit i % 16 of keys i / 16 and i / 16 + 32);
-//    one barrier per tile.
+//  * pipeline: BA_NBUF LDS tile buffers filled by DMA; waves 0-3 run a step as O update of the
+//    previous tile, S' and softmax of this one, waves 4-7 (on the same SIMDs) half a step behind, so
+//    that one wave's MFMAs meet the other's softmax; one barrier per tile.
 // Numerics against the math path: every p is one bf16 rounding of a probability scaled by at
 // most 2^TAU, and the running rescale is exact up to fp32 rounding, as in any online softmax.
 // Writes (m, l, acc) partials per (query row, head, split) -- m in natural-log units, as

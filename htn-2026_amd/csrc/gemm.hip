@@ -547,9 +547,6 @@ static void stream_go(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, i
       x, xs, (int)M, w, (int)N, (int)K, out, os, res, rs, pval, pidx, logits);
 }
 
-// Passes of G tiles from the units per workgroup: o / down (10 units at 256 CUs) one tile,
-// qkv (24) two, gate/up (38 act rows) three gate + three up tiles (two at 64 rows, where the
-// activation tiles take the LDS), the LM head (594) four per pass.
 // The LM head: four 16-row tiles per pass (~600 rows per workgroup at 256 CUs).
 template <int MT, int EPI>
 static int64_t stream_mt(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N,

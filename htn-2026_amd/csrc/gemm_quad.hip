@@ -1,6 +1,7 @@
-// Four-wave MFMA GEMM for 257 and more activation rows (prefill chunks), and the LM head over 129
-// and more:  out[m, n] = epi( sum_k X[m, k] * W[n, k] )  (the reference's cuBLAS prefill,
-// engine.py:550-592, and its tensor-core GEMMs, gemv.py:61-116, at many rows).
+// Four-wave MFMA GEMM:  out[m, n] = epi( sum_k X[m, k] * W[n, k] )  for 257 and more activation rows
+// (prefill chunks) and for 33 to 64 (mid-sized batches, small trees), the split partials of decode steps
+// of 65 to 128 rows, and the LM head over 33 to 64 and 129 and more  (the reference's cuBLAS prefill,
+// engine.py:550-592, and its tensor-core GEMMs, gemv.py:61-116).
 //
 // A workgroup of 4 waves, one per SIMD, owns 32 MT activation rows x 32 NT weight rows (SwiGLU: 16 NT gate
 // and the 16 NT up rows of the same outputs); wave (wm, wn) the quarter of 16 MT x 16 NT, MT x NT
@@ -26,7 +27,7 @@
 //    one XCD runs at a time (4 row blocks x 8 weight blocks) cover theirs once.  gate/up at 16384
 //    rows 1356 -> 1243 us, 512 rows (128 x 160 pairs) 69 -> 58 us; with three and more buffers it
 //    gains nothing.
-//  * Weight rows enter the MFMA tiles pairwise interleaved (frag_row): the lane then holds eight
+//  * Weight rows enter the MFMA tiles pairwise interleaved (rd): the lane then holds eight
 //    consecutive output columns of a tile pair, one 16-byte store per row instead of two 8-byte
 //    stores in different lines.
 // The accumulation of an output runs through its K range in order, 32 at a time: the bits are the
@@ -358,8 +359,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
 // Tile shapes {MT, NT, stage buffers} and the time of one round of workgroups over the CUs,
 // a + b x stages (SwiGLU: + QUAD_SWIGLU MT NT) in us: least squares over 14 row counts from 300 to
 // 16384 x the four Qwen3-4B projections x every shape on MI355X, weights from HBM (single launches
-// scatter by about 8 %).  The plan takes the shape whose rounds cost least; over those launches
-// its choice is 0.4 % off the best measured shape on average, 11 % at most.  Times (us) with the
+// scatter by about 8 %).  The plan takes the shape whose rounds cost least.  Times (us) with the
 // kernels before (8 waves, 128 x 128 tiles to 1023 rows, 256 x 256 from 1024) -> now, o and down
 // at 512 rows with their split reduce:
 //   rows    qkv (6144 x 2560)  o (2560 x 4096)  gate/up (19456 x 2560)  down (2560 x 9728)
@@ -367,9 +367,10 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
 //   1024       64.9 ->  35.7     93.9 ->  32.2     135.1 ->  115.4       206.8 ->  70.7
 //   3000      123.0 ->  88.9     96.6 ->  56.6     266.8 ->  261.4       206.2 -> 119.2
 //   16384     418.3 -> 393.4    313.2 -> 293.7    1342.0 -> 1265.2       716.4 -> 657.9
-// (the whole-round rates at 16384 rows are 1.17 to 1.31 PFLOP/s.)  Without its loads the 8 x 8
-// loop runs at 1.52 to 1.56 PFLOP/s: what is left is a round's start and end, when the first
-// lines come from HBM and the outputs are written with no MFMAs beside them (11 to 17 us).
+// (the whole-round rates at 16384 rows are 1.17 to 1.31 PFLOP/s, the matrix cores 58 to 70 % busy at
+// 32768.)  What is left is the line stream, a fifth of it past the L2, and a round's start and end,
+// when the first lines come from HBM and the outputs are written with no MFMAs beside them (the
+// fitted a: 4 to 13 us).
 struct QuadShape {
   int mt, nt, nbuf;
   float a, b;
@@ -590,7 +591,7 @@ int64_t quad_small_ws_floats(int64_t M, int64_t N, int64_t K) {
 // block of vocabulary rows; the last block may pass the vocabulary: its missing rows reload a valid
 // one and are never ranked); 0, with nothing launched, for other shapes.  129 and more rows: 256 x
 // 256 tiles.  33..64 rows: 320 vocabulary rows per workgroup, two nearly full rounds (475
-// workgroups at 151936), 64 KiB of weights in flight per CU: 40 rows 275 -> 138 us (5.6 TB/s) against
+// workgroups at 151936), three stages of 40 KiB of weights in LDS: 40 rows 275 -> 138 us (5.6 TB/s) against
 // gemm_stream_kernel, which re-stages the activations with every chunk; 64 rows 285 -> 139 us
 // ({2, 4} tiles 139 / 146, {2, 8} 157 / 159).  65..128 rows stay on gemm_tile_kernel: 167 us at
 // 100 rows against 174 with {4, 8} tiles here.

@@ -1,5 +1,7 @@
-// LDS-tiled MFMA GEMM for many activation rows (tree verification B*T rows, prefill chunks):
-//   out[m, n] = epi( sum_k X[m, k] * W[n, k] )
+// MFMA GEMMs for many activation rows:  out[m, n] = epi( sum_k X[m, k] * W[n, k] )
+// gemm_rows_kernel (below): 65 to 256 rows (tree verification).  gemm_tile_kernel, here: the LM head
+// over 65 to 128 rows, and products whose 32-bit offsets neither it nor the four-wave kernel reach
+// (rows or weights of 4 GiB and more); the dispatch to gemm_quad.hip and the split reduction sit here too,
 // with the epilogues of the decode GEMM (store / residual / SwiGLU / per-tile argmax for the LM
 // head) -- the large-M counterpart of the reference's tensor-core GEMMs (gemv.py:61-116 with
 // BLOCK_M >= 16, fast.py:161-213) and of its cuBLAS prefill (engine.py:550-592).

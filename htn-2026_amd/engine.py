@@ -35,7 +35,7 @@ DEVICE = os.environ.get("ENGINE_DEVICE", "cuda:0")
 TREE_MODE = os.environ.get("ENGINE_TREE", "auto")
 TREE_CHECK_TOKENS = 128   # tokens the gate generates each way (engine.py:88)
 TREE_MIN_GAIN = 0.92      # keep trees only below this fraction of the plain wall time (engine.py:89)
-TREE_MAX_ROWS = 64        # verification rows B * T: the weight-streaming GEMM regime
+TREE_MAX_ROWS = 64        # verification rows B * T: where the weight stream is the cost
 
 
 class _Shape:

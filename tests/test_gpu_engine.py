@@ -143,7 +143,7 @@ def test_generate_resets_state_and_is_deterministic(eng4):
 
 def test_prefill_chunking_is_invariant(eng4, ref4):
     """Chunks of 7 / 64 / 96 tokens per sequence run the projections through different GEMM
-    kernels (LDS-staged for <= 64 rows, register-blocked above), whose fp32 summation orders
+    kernels (skinny, all-rows, four-wave), whose fp32 summation orders
     differ in the last bits: every chunking must emit a greedy decode under the margin rule, and
     the chunkings must agree on every step before a row's first oracle tie."""
     say("prefill chunk sizes 7 / 64 / whole prompt: same ids up to oracle ties")
@@ -197,8 +197,8 @@ def ref2():
 
 @pytest.mark.parametrize("B,S,N", [(2, 33, 8), (5, 40, 6), (32, 64, 6), (64, 24, 4), (80, 16, 4)])
 def test_batched_decode_paths(eng2, ref2, B, S, N):
-    """Vector path B <= 2; LDS-staged MFMA GEMMs + streaming LM head 3..64 rows (16-, 32- and
-    two 32-row activation tiles); the tiled GEMMs past 64 rows."""
+    """Vector path B <= 2; skinny MFMA GEMMs 3..32 rows; four-wave GEMMs at 64; all-rows GEMMs past
+    that."""
     say(f"batched decode B={B} S={S} N={N}")
     prompt = synth.prompt_ids(20 + B, B, S)
     toks = np.array(list(eng2.generate(prompt.tolist(), N))).T
