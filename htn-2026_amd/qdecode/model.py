@@ -375,7 +375,7 @@ class BlockRunner:
 # Measured on MI355X (prefill + first token, second of three runs): 4 x 8192 0.330 s (6144 rows:
 # 0.342, 8192: 0.356, 12288: 0.335, 16384: 0.330, 24576: 0.336); 32 x 2048 0.515 s (6144: 0.541,
 # 8192: 0.578, 12288: 0.521, 16384: 0.527, 24576: 0.524).  The block step's buffers grow with it
-# (1.91 GB of activations at 32768 rows; its workspace stays at ~34 MB whatever the context).
+# (1.91 GB of activations at 32768 rows; its workspace stays at ~50 MB whatever the context).
 PREFILL_ROWS = 32768
 
 
