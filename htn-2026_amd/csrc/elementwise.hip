@@ -886,14 +886,15 @@ void launch_read_probe(const void* buf, int64_t bytes, int grid, uint32_t* sink,
 // ------------------------------------------------------------------ greedy argmax reduction
 // tok[m] = index of the maximum over the per-tile (value, lowest index) partials of row m,
 // lowest index on exact ties (gemv.py:147-154, fast.py:402-426); optionally pos[0] += 1.
-// One workgroup per row, a latency chain and nothing else: eight partials per thread are requested
-// before the first is compared, waves meet through registers and one barrier.  Measured with the
-// LM head of one row (4748 partials): 9.1 -> 5.6 us (475 partials of 40 rows: 4.6, unchanged).
+// One workgroup per row, a latency chain and nothing else: U partials per thread are requested before
+// the first is compared, waves meet through registers and one barrier.  Measured with the LM head of
+// one row (4748 partials, U = 8): 9.1 -> 5.6 us.  Up to 256 and 512 partials U is 1 and 2: more would
+// only repeat loads (LM head of 129 rows over 1000: 21.5 us with 8, 20.2).
+template <int U>
 __global__ __launch_bounds__(256) void argmax_reduce_kernel(const float* __restrict__ pval,
                                                             const int32_t* __restrict__ pidx,
                                                             int64_t nparts, int64_t* tok,
                                                             int64_t* pos_inc) {
-  constexpr int U = 8;
   __shared__ float sv[4];
   __shared__ int32_t si[4];
   const int64_t m = blockIdx.x;
@@ -938,5 +939,8 @@ __global__ __launch_bounds__(256) void argmax_reduce_kernel(const float* __restr
 void launch_argmax_reduce(const float* pval, const int32_t* pidx, int64_t nparts, int64_t M,
                           int64_t* tok, int64_t* pos_inc, hipStream_t s) {
   if (M <= 0) return;
-  argmax_reduce_kernel<<<dim3((unsigned)M), dim3(256), 0, s>>>(pval, pidx, nparts, tok, pos_inc);
+  const dim3 g((unsigned)M), b(256);
+  if (nparts <= 256) argmax_reduce_kernel<1><<<g, b, 0, s>>>(pval, pidx, nparts, tok, pos_inc);
+  else if (nparts <= 512) argmax_reduce_kernel<2><<<g, b, 0, s>>>(pval, pidx, nparts, tok, pos_inc);
+  else argmax_reduce_kernel<8><<<g, b, 0, s>>>(pval, pidx, nparts, tok, pos_inc);
 }
