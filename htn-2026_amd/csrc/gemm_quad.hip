@@ -397,16 +397,20 @@ static_assert(quad_fits(), "the CU's LDS");
 // (gemm_tile_splits), one round of {4, 4}.
 constexpr int QUAD_SPLIT = 2;
 
+// us of a launch in shape q
+double quad_cost(const QuadShape& q, int64_t M, int64_t N, bool sw, int64_t splits, int64_t stages) {
+  const int64_t bm = 32 * q.mt, bn = quad_outs(q.nt, sw);
+  const int64_t wgs = (M + bm - 1) / bm * ((N + bn - 1) / bn) * splits;
+  return (double)((wgs + plan_cus() - 1) / plan_cus()) *
+         (q.a + (sw ? QUAD_SWIGLU * q.mt * q.nt : 0.0) + (double)q.b * stages);
+}
+
 int quad_plan(int64_t M, int64_t N, bool sw, int64_t splits, int64_t stages) {
   int best = -1;
   double best_t = 0;
   for (int i = 0; i < (splits > 1 ? QUAD_SPLIT : QUADS); ++i) {
-    const QuadShape& q = QUAD[i];
-    if (sw && q.nt % 2) continue;
-    const int64_t bm = 32 * q.mt, bn = quad_outs(q.nt, sw);
-    const int64_t wgs = (M + bm - 1) / bm * ((N + bn - 1) / bn) * splits;
-    const double t = (double)((wgs + plan_cus() - 1) / plan_cus()) *
-                     (q.a + (sw ? QUAD_SWIGLU * q.mt * q.nt : 0.0) + (double)q.b * stages);
+    if (sw && QUAD[i].nt % 2) continue;
+    const double t = quad_cost(QUAD[i], M, N, sw, splits, stages);
     if (best < 0 || t < best_t) {
       best = i;
       best_t = t;
@@ -589,12 +593,26 @@ int64_t quad_small_ws_floats(int64_t M, int64_t N, int64_t K) {
 
 // LM head over 33..64 and 129 and more rows: argmax partials pval / pidx [M][return value] (one per
 // block of vocabulary rows; the last block may pass the vocabulary: its missing rows reload a valid
-// one and are never ranked); 0, with nothing launched, for other shapes.  129 and more rows: 256 x
-// 256 tiles.  33..64 rows: 320 vocabulary rows per workgroup, two nearly full rounds (475
-// workgroups at 151936), three stages of 40 KiB of weights in LDS: 40 rows 275 -> 138 us (5.6 TB/s) against
-// gemm_stream_kernel, which re-stages the activations with every chunk; 64 rows 285 -> 139 us
-// ({2, 4} tiles 139 / 146, {2, 8} 157 / 159).  65..128 rows stay on gemm_tile_kernel: 167 us at
-// 100 rows against 174 with {4, 8} tiles here.
+// one and are never ranked); 0, with nothing launched, for other shapes.  129 and more rows: of three
+// tile shapes the one that the cost above favours; with {8, 8} alone, 256 rows, the whole head over 129
+// rows took 252 us at 151936 (8-wave kernel 246; {6, 8}: 239) and 62.9 at 16000 (60.0; {4, 4}: 31.7).
+// 33..64 rows: 320 vocabulary rows per workgroup, two nearly full rounds (475 workgroups at 151936), three
+// stages of 40 KiB of weights in LDS: 40 rows 275 -> 138 us (5.6 TB/s) against gemm_stream_kernel, which
+// re-stages the activations with every chunk; 64 rows 285 -> 139 us ({2, 4} tiles 139 / 146, {2, 8} 157 /
+// 159).  Under LM_SMALL_BLOCKS workgroups the stream kernel's 256 are faster (33 rows at 8192: 33.8 against
+// 35.9).  65..128 rows stay on gemm_tile_kernel: 167 us at 100 rows against 174 with {4, 8} tiles here.
+constexpr int64_t LM_SMALL_BLOCKS = 48;
+
+template <int MT, int NT, int NBUF>
+static int64_t lm_quad_go(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
+                          float* pval, int32_t* pidx, float* logits, hipStream_t s) {
+  const int64_t mbl = (M + 32 * MT - 1) / (32 * MT), nbl = (N + 32 * NT - 1) / (32 * NT);
+  gemm_quad_kernel<EPI_ARGMAX, false, MT, NT, NBUF><<<dim3((unsigned)(mbl * nbl)), dim3(256), 0, s>>>(
+      x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, 32 * NT, (int)(K / TK), nullptr, 0, nullptr, 0, 0,
+      nullptr, pval, pidx, logits);
+  return nbl;
+}
+
 int64_t launch_lm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
                        float* pval, int32_t* pidx, float* logits, hipStream_t s) {
   const bool small = M >= 33 && M <= 64;
@@ -602,14 +620,15 @@ int64_t launch_lm_quad(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
       !quad_offsets_ok(xs, N, K, EPI_ARGMAX))
     return 0;
   if (xs % 8 || reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16) return 0;
-  const int64_t bm = small ? 64 : 256, bn = small ? 320 : 256;
-  const int64_t mbl = (M + bm - 1) / bm, nbl = (N + bn - 1) / bn;
-#define QD_LM(MT, NT, NB)                                                                       \
-  gemm_quad_kernel<EPI_ARGMAX, false, MT, NT, NB><<<dim3((unsigned)(mbl * nbl)), dim3(256), 0, s>>>( \
-      x, xs, (int)M, w, (int)N, (int)K, (int)mbl, (int)nbl, (int)bn, (int)(K / TK), nullptr, 0, nullptr, \
-      0, 0, nullptr, pval, pidx, logits)
-  if (small) QD_LM(2, 10, 3);
-  else QD_LM(8, 8, 2);
-#undef QD_LM
-  return nbl;
+  if (small) {
+    if ((N + 319) / 320 < LM_SMALL_BLOCKS) return 0;
+    return lm_quad_go<2, 10, 3>(x, xs, M, w, N, K, pval, pidx, logits, s);
+  }
+  constexpr QuadShape S0 = QUAD[1], S1 = QUAD[8], S2 = QUAD[12];
+  static_assert(S0.nt % 2 == 0 && S1.mt == 6 && S1.nt == 8 && S2.mt == 8, "{4, 4}, {6, 8}, {8, 8}");
+  const double t0 = quad_cost(S0, M, N, false, 1, K / TK), t1 = quad_cost(S1, M, N, false, 1, K / TK),
+               t2 = quad_cost(S2, M, N, false, 1, K / TK);
+  if (t0 < t1 && t0 < t2) return lm_quad_go<S0.mt, S0.nt, S0.nbuf>(x, xs, M, w, N, K, pval, pidx, logits, s);
+  if (t1 < t2) return lm_quad_go<S1.mt, S1.nt, S1.nbuf>(x, xs, M, w, N, K, pval, pidx, logits, s);
+  return lm_quad_go<S2.mt, S2.nt, S2.nbuf>(x, xs, M, w, N, K, pval, pidx, logits, s);
 }

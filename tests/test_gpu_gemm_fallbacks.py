@@ -75,3 +75,11 @@ def test_lm_head_vocabularies_at_33_to_64_rows(ops, M, V, K):
     want = ops.rmsnorm(x, nw, 1e-6).double() @ w.double().t()
     assert float((logits.double() - want).abs().max()) <= 1e-4
     assert torch.equal(tok.cpu(), torch.argmax(logits.to(BF).float().cpu(), dim=-1))
+
+
+# the vocabularies from which 33 to 64 rows take the four-wave kernel (48 blocks of 320), and the tile
+# shapes of 129 rows and more
+@pytest.mark.parametrize("M,V", [(33, 15040), (64, 15044), (129, 256), (129, 16000), (192, 40064), (193, 40064),
+                                 (257, 33152)])
+def test_lm_head_tile_shapes(ops, M, V):
+    test_lm_head_vocabularies_at_33_to_64_rows(ops, M, V, 1024)
