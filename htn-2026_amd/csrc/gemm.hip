@@ -563,7 +563,8 @@ static int64_t gemm_mt(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
                        float* pval, int32_t* pidx, float* logits, float* part, int64_t part_floats,
                        hipStream_t s) {
   if (M >= (EPI == EPI_ARGMAX ? GEMM_TILE_MIN_M : GEMM_SMALL_MIN_M) &&
-      gemm_tile_ok(M, N, K, EPI, x, xs, w, out, os, res, rs))
+      gemm_tile_ok(M, N, K, EPI, x, xs, w, out, os, res, rs) &&
+      (M >= GEMM_TILE_MIN_M || quad_small_pays(M, N, K, EPI, part ? part_floats : 0)))
     return launch_gemm_tile(x, xs, M, w, N, K, out, os, res, rs, EPI, pval, pidx, logits, part,
                             part_floats, s);
   const int P = stream_grid();
@@ -571,8 +572,9 @@ static int64_t gemm_mt(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, 
                        reinterpret_cast<uintptr_t>(w) % 16 == 0;
   // the LM head: 3..32 rows on the skinny argmax kernel (activations resident in LDS per K
   // phase); 33..64 rows on the four-wave kernel; the projections: 3..32 rows on the skinny kernel,
-  // 33..64 on the four-wave one.  What those do not take (unaligned operands, odd widths): the
-  // weight-streaming and LDS-staged kernels here
+  // 33..64 on the four-wave one.  What those do not take (unaligned operands, odd widths) and where
+  // they do not pay (narrow products, small vocabularies): the weight-streaming and LDS-staged kernels
+  // here
   if constexpr (EPI == EPI_ARGMAX) {
     if (M <= 32) {
       const int64_t parts = launch_lm_skinny(x, xs, M, w, N, K, pval, pidx, logits, s);

@@ -540,6 +540,24 @@ static void quad_small_go(const SmallPlan& P, const bf16_t* x, int64_t xs, int64
 #undef QD_SMALL
 }
 
+// Whether a whole product of 33..64 rows is faster here than on gemm_lds_kernel (K a multiple of 512),
+// whose workgroups of 16 columns split K over their waves: up to 2048 columns they are one round of the
+// CUs, and its time hardly grows with K, while a workgroup here walks its K range stage by stage.  Past
+// 2048 columns always.  Up to there the K splits win from K = 2048 on (to 2560: up to 1024 columns); SwiGLU, or
+// a product without room for partials, has none.  33 rows, weights from HBM (us, there -> here):
+//   N x K                 store, split       store, no room     SwiGLU (2N weight rows)
+//   512 x 512             3.4 -> 5.7         3.4 -> 4.2          4.5 ->  4.8
+//   2048 x 1024           5.1 -> 6.5         5.1 -> 6.2          7.5 ->  7.0
+//   1024 x 2560           7.4 -> 6.9         7.4 -> 10.9        10.0 -> 12.0
+//   2048 x 2560           8.1 -> 8.0 (64 rows 8.6 -> 8.9)  8.1 -> 11.2   11.7 -> 12.4
+//   1024 x 8192          15.1 -> 9.7        15.1 -> 27.2        21.8 -> 29.6
+//   3072 x 1024           8.2 -> 7.1         8.2 ->  6.3        11.6 ->  7.3
+bool quad_small_pays(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats) {
+  if (K % 512 || N > 2048) return true;
+  if (epi == EPI_SWIGLU) return K < 1536 && N > K;
+  return part_floats >= 2 * M * N && K > 1536 && (K > 2560 || N <= 1024);
+}
+
 // The operands satisfy gemm_tile_ok, 33 <= M <= 64 (quad_small_partials: 128).  quad_small_partials: fp32 partials
 // part[S][M][N], S returned (0, nothing launched: no split fits part_floats or pays).
 // launch_quad_small: the whole product; with splits its partials go to part, their count is

@@ -775,6 +775,7 @@ int gemm_quad_query(int64_t M, int64_t N, int64_t K, int epi, int64_t part_float
   RowsPlan P;
   if (M < GEMM_SMALL_MIN_M || !gemm_tile_ok(M, N, K, epi, a, K, a, a, N, a, N)) return 0;
   if (M < GEMM_TILE_MIN_M) {
+    if (!quad_small_pays(M, N, K, epi, part_floats)) return 0;
     quad_small_query(M, N, K, epi, part_floats, out);
     return 1;
   }

@@ -131,6 +131,7 @@ int quad_small_partials(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w,
 int launch_quad_small(const bf16_t* x, int64_t xs, int64_t M, const bf16_t* w, int64_t N, int64_t K,
                       bf16_t* out, int64_t os, const bf16_t* res, int64_t rs, int epi, float* part,
                       int64_t part_floats, hipStream_t s);
+bool quad_small_pays(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats);
 int64_t quad_small_ws_floats(int64_t M, int64_t N, int64_t K);
 void quad_query(int64_t M, int64_t N, int64_t K, int epi, int splits, int ks_per, int64_t* out);
 void quad_small_query(int64_t M, int64_t N, int64_t K, int epi, int64_t part_floats, int64_t* out);

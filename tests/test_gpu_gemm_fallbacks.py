@@ -48,6 +48,21 @@ def test_widths_at_33_to_64_rows(ops, M, N, K, epi):
     check_linear(ops, epi, x, N, g)
 
 
+# on both sides of the columns and K at which whole products of 33 to 64 rows stay on the LDS-staged
+# kernel, with room for split partials and without
+@pytest.mark.parametrize("epi", [0, 1, 2])
+@pytest.mark.parametrize("N,K", [(128, 512), (1024, 1024), (2048, 1536), (2048, 2048), (1024, 2560), (1152, 2560),
+                                 (2048, 4096), (2176, 1024)])
+@pytest.mark.parametrize("M", [33, 64])
+def test_narrow_products_at_33_to_64_rows(ops, M, N, K, epi):
+    print(f"\n[case] {M} x {N} x {K}, epilogue {epi}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K + epi)
+    x = torch.empty((M, K), dtype=BF, device="cuda").normal_(0, 1, generator=g)
+    check_linear(ops, epi, x, N, g)
+    check_linear(ops, epi, x, N, g, ws=torch.zeros(256, dtype=torch.uint8, device="cuda"))
+
+
 @pytest.mark.parametrize("M", [33, 64])
 def test_unaligned_output_at_33_to_64_rows(ops, M):
     """Output rows that start 2 bytes off: not the four-wave kernel's 8-byte stores."""

@@ -57,6 +57,9 @@ def test_plans_cover_their_product(plan):
                 for epi in (0, 1, 2):
                     for room in (0, 3 * M * N, ROOM):
                         p = plan(M, N, K, epi, room)
+                        if p is None:            # the LDS-staged kernel's
+                            assert M <= 64 and N <= 2048 and K % 512 == 0
+                            continue
                         kind, mt, nt = p["key"]
                         S, ks = p["splits"], p["ks_per"]
                         assert (S - 1) * ks < K // 64 <= S * ks
