@@ -359,7 +359,8 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(
 // Tile shapes {MT, NT, stage buffers} and the time of one round of workgroups over the CUs,
 // a + b x stages (SwiGLU: + QUAD_SWIGLU MT NT) in us: least squares over 14 row counts from 300 to
 // 16384 x the four Qwen3-4B projections x every shape on MI355X, weights from HBM (single launches
-// scatter by about 8 %).  The plan takes the shape whose rounds cost least.  Times (us) with the
+// scatter by about 8 %).  The plan takes the shape whose rounds cost least: over 78 launches of other
+// sizes the fastest shape in 61, 0.4 % off it on average, 5.8 % at most.  Times (us) with the
 // kernels before (8 waves, 128 x 128 tiles to 1023 rows, 256 x 256 from 1024) -> now, o and down
 // at 512 rows with their split reduce:
 //   rows    qkv (6144 x 2560)  o (2560 x 4096)  gate/up (19456 x 2560)  down (2560 x 9728)
